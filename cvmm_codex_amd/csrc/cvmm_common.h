@@ -117,6 +117,24 @@ __device__ __forceinline__ int64_t wave_incl_scan(int64_t v) {
   return v;
 }
 
+// 32-bit inclusive scan by DPP row shifts and broadcasts (no LDS crossbar):
+// shifts by 1, 2, 4, 8 within each row of 16 lanes, then row 0's (2's) last
+// lane to row 1 (3), then lane 31 to rows 2 and 3.
+__device__ __forceinline__ int32_t wave_incl_scan(int32_t v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+  return v;
+}
+
+// The wave's sum, as a scalar.
+__device__ __forceinline__ int32_t wave_sum(int32_t v) {
+  return __builtin_amdgcn_readlane(wave_incl_scan(v), 63);
+}
+
 // Workgroup barrier for a hand-over through LDS only: this wave's LDS
 // operations complete (lgkmcnt(0)), then s_barrier.  __syncthreads() would
 // also wait for the wave's outstanding global stores (its release fence),
@@ -190,6 +208,13 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t i, int64_t n) {
   const int64_t xcd = i % kXcd, local = i / kXcd;
   const int64_t per = n / kXcd, rem = n % kXcd;
   return xcd * per + (xcd < rem ? xcd : rem) + local;
+}
+
+// 32-bit form of the above for the routed GEMMs' tiles.
+__device__ __forceinline__ uint32_t xcd_remap(uint32_t i, uint32_t n) {
+  if (n < 8) return i;
+  const uint32_t xcd = i % 8, per = n / 8, rem = n % 8;
+  return xcd * per + (xcd < rem ? xcd : rem) + i / 8;
 }
 
 }  // namespace cvmm

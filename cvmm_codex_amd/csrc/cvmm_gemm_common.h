@@ -29,105 +29,146 @@ struct RouteMeta {
   int64_t dgrow[BM];  // x row for the routing-weight gradient
   float w[BM];        // rounded routing weight (1 if unweighted)
   int32_t expert;
+  int32_t tile, group;  // the workgroup's m-tile and column group
   int64_t row0;
   int32_t rows;
 };
 
-// Find the (expert, first route, row count) of m-tile `tile`: expert e owns
-// ceil(count_e / BM) consecutive tiles.  Wave 0 scans the offsets 64 experts at
-// a time; returns false (uniformly) when `tile` is past the last tile.
-template <int BM>
-__device__ bool gemm_schedule_tile(const GemmParams& p, int64_t tile, RouteMeta<BM>& m) {
+// A value every lane holds, as a scalar.
+__device__ __forceinline__ int32_t uniform_i32(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// The m-tile and column group of this workgroup, and the tile's (expert, first
+// route, row count): expert e owns ceil(count_e / BM) tiles.  Workgroups of
+// one m-tile are `n_groups` column groups.  Returns false (uniformly) for a
+// workgroup past the last m-tile.
+//
+// The launch holds R / BM + E tiles, the most there can be; the real count
+// follows from the offsets.  Only the real tiles are spread over the XCDs
+// (contiguous runs, equal shares), with the surplus workgroups after them:
+// spreading the launched grid instead gave the last XCDs nothing but surplus
+// (one XCD in eight at 12 % surplus, three where the average expert holds
+// under one tile).  Same-box steps, grid spread -> this: 32 decoded tokens
+// over 128 experts 676 -> 627 us, a 1999-token prefill 753 -> 739, the FFN
+// stack's training step 3630 -> 3574, ff_up and ff_down unchanged (one
+// round of tiles either way).  XCD false: ids in launch order.
+template <int BM, bool XCD = true>
+__device__ bool gemm_schedule_tile(const GemmParams& p, int64_t n_groups, RouteMeta<BM>& m) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  // ---- schedule: which expert / routes does m-tile `tile` cover? -----------
-  if (wave == 0 && p.token_major > 0) {
-    // Token-major order: all tiles with index j within their expert, in
-    // expert order, then index j + 1.  Routes of an expert are sorted by
-    // token, so tile j of every expert covers about the same token range and
-    // neighbouring workgroups (one XCD) gather the same activation rows.
-    // C(j) = sum_e min(nt_e, j) tiles come before index j; binary search.
+  if (wave == 0) {
     constexpr int G = kTokenMajorMaxExperts / 64;
     if (lane == 0) m.expert = -1;
-    int64_t st[G], en[G], nt[G], ntmax = 0;
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const int32_t e = g * 64 + lane;
-      st[g] = en[g] = nt[g] = 0;
+    // the routes [st, en) of expert e (none past the last expert)
+    auto range = [&](int32_t e, int64_t& st, int64_t& en) {
+      st = en = 0;
       if (e < p.n_experts) {
         int64_t end = p.offsets[e];
         int64_t start = e > 0 ? p.offsets[e - 1] : 0;
         end = end < 0 ? 0 : (end > p.n_routes ? p.n_routes : end);
         start = start < 0 ? 0 : (start > p.n_routes ? p.n_routes : start);
         if (end < start) end = start;
-        st[g] = start;
-        en[g] = end;
-        nt[g] = (end - start + BM - 1) / BM;
+        st = start;
+        en = end;
       }
-      ntmax = nt[g] > ntmax ? nt[g] : ntmax;
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-      const int64_t v = __shfl_xor(ntmax, o, 64);
-      ntmax = v > ntmax ? v : ntmax;
-    }
-    auto before = [&](int64_t j) {
-      int64_t s = 0;
-#pragma unroll
-      for (int g = 0; g < G; ++g) s += nt[g] < j ? nt[g] : j;
-      return __shfl(wave_incl_scan(s), 63, 64);
     };
-    const int64_t n_tiles = before(ntmax);
-    if (lane == 0 && tile >= n_tiles) m.row0 = n_tiles;  // past the last tile: the tile count
-    if (tile < n_tiles) {
-      int64_t lo = 0, hi = ntmax;  // before(lo) <= tile < before(hi)
-      while (hi - lo > 1) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (before(mid) <= tile) lo = mid;
-        else hi = mid;
+    auto tiles_of = [](int64_t st, int64_t en) { return (int32_t)((en - st + BM - 1) / BM); };
+    auto place = [&](int32_t e, int64_t r0, int64_t end) {
+      m.expert = e;
+      m.row0 = r0;
+      m.rows = (int32_t)((end - r0) < BM ? (end - r0) : BM);
+    };
+    int32_t tile = 0, n_tiles = 0;
+    // this workgroup's m-tile among the real ones (the launch's workgroup
+    // count fits 31 bits)
+    auto locate = [&]() {
+      const uint32_t ng = (uint32_t)n_groups, n_real = (uint32_t)n_tiles * ng;
+      const uint32_t i = blockIdx.x;
+      const uint32_t id = XCD && i < n_real ? xcd_remap(i, n_real) : i;
+      tile = (int32_t)(id / ng);
+      if (lane == 0) {
+        m.tile = tile;
+        m.group = (int32_t)(id - (uint32_t)tile * ng);
+        if (tile >= n_tiles) m.row0 = n_tiles;  // past the last tile: the tile count
       }
-      int64_t r = tile - before(lo);  // rank among the experts with more than lo tiles
-      const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    };
+    if (p.n_experts <= kTokenMajorMaxExperts) {
+      int64_t st[G], en[G];
+      int32_t nt[G], incl[G], ntmax = 0;
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        const bool has = nt[g] > lo;
-        const uint64_t b = __ballot(has);
-        const int64_t cnt = __popcll(b);
-        if (r >= 0 && r < cnt && has && (int64_t)__popcll(b & lt_mask) == r) {
-          m.expert = g * 64 + lane;
-          const int64_t r0 = st[g] + lo * BM;
-          m.row0 = r0;
-          m.rows = (int32_t)((en[g] - r0) < BM ? (en[g] - r0) : BM);
+        range(g * 64 + lane, st[g], en[g]);
+        nt[g] = tiles_of(st[g], en[g]);
+        ntmax = nt[g] > ntmax ? nt[g] : ntmax;
+      }
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        incl[g] = wave_incl_scan(nt[g]) + n_tiles;
+        n_tiles = __builtin_amdgcn_readlane(incl[g], 63);
+      }
+      locate();
+      if (tile < n_tiles && p.token_major > 0) {
+        // Token-major order: all tiles with index j within their expert, in
+        // expert order, then index j + 1.  Routes of an expert are sorted by
+        // token, so tile j of every expert covers about the same token range
+        // and neighbouring workgroups (one XCD) gather the same activation
+        // rows.  C(j) = sum_e min(nt_e, j) tiles come before index j; binary
+        // search.
+        for (int o = 32; o > 0; o >>= 1) {
+          const int32_t v = __shfl_xor(ntmax, o, 64);
+          ntmax = v > ntmax ? v : ntmax;
         }
-        r -= cnt;
+        auto before = [&](int32_t j) {
+          int32_t s = 0;
+#pragma unroll
+          for (int g = 0; g < G; ++g) s += nt[g] < j ? nt[g] : j;
+          return wave_sum(s);
+        };
+        int32_t lo = 0, hi = ntmax;  // before(lo) <= tile < before(hi)
+        while (hi - lo > 1) {
+          const int32_t mid = (lo + hi) >> 1;
+          if (before(mid) <= tile) lo = mid;
+          else hi = mid;
+        }
+        int32_t r = tile - before(lo);  // rank among the experts with more than lo tiles
+        const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const bool has = nt[g] > lo;
+          const uint64_t b = __ballot(has);
+          const int32_t cnt = __popcll(b);
+          if (r >= 0 && r < cnt && has && (int32_t)__popcll(b & lt_mask) == r)
+            place(g * 64 + lane, st[g] + (int64_t)lo * BM, en[g]);
+          r -= cnt;
+        }
+      } else if (tile < n_tiles) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const int32_t excl = incl[g] - nt[g];
+          if (tile >= excl && tile < incl[g]) place(g * 64 + lane, st[g] + (int64_t)(tile - excl) * BM, en[g]);
+        }
+      }
+    } else {
+      // more experts than the registers hold: one pass for the tile count,
+      // one for the tile
+      int32_t sum = 0;
+      int64_t st, en;
+      for (int32_t base = 0; base < p.n_experts; base += 64) {
+        range(base + lane, st, en);
+        sum += tiles_of(st, en);
+      }
+      n_tiles = wave_sum(sum);
+      locate();
+      int32_t carry = 0;
+      for (int32_t base = 0; tile < n_tiles && base < p.n_experts; base += 64) {
+        range(base + lane, st, en);
+        const int32_t nt = tiles_of(st, en);
+        const int32_t incl = wave_incl_scan(nt) + carry, excl = incl - nt;
+        if (tile >= excl && tile < incl) place(base + lane, st + (int64_t)(tile - excl) * BM, en);
+        carry = __builtin_amdgcn_readlane(incl, 63);
+        if (tile < carry) break;
       }
     }
-  } else if (wave == 0) {
-    if (lane == 0) m.expert = -1;
-    int64_t carry = 0;
-    for (int32_t base = 0; base < p.n_experts; base += 64) {
-      const int32_t e = base + lane;
-      int64_t start = 0, end = 0;
-      if (e < p.n_experts) {
-        end = p.offsets[e];
-        start = e > 0 ? p.offsets[e - 1] : 0;
-        end = end < 0 ? 0 : (end > p.n_routes ? p.n_routes : end);
-        start = start < 0 ? 0 : (start > p.n_routes ? p.n_routes : start);
-        if (end < start) end = start;
-      }
-      const int64_t nt = (end - start + BM - 1) / BM;
-      const int64_t incl = wave_incl_scan(nt) + carry;
-      const int64_t excl = incl - nt;
-      if (e < p.n_experts && tile >= excl && tile < incl) {
-        m.expert = e;
-        const int64_t r0 = start + (tile - excl) * BM;
-        m.row0 = r0;
-        m.rows = (int32_t)((end - r0) < BM ? (end - r0) : BM);
-      }
-      carry = __shfl(incl, 63, 64);
-      if (tile < carry) break;
-    }
-    if (lane == 0 && m.expert < 0) m.row0 = carry;  // past the last tile: the tile count
   }
   __syncthreads();
   return m.expert >= 0;
@@ -170,8 +211,8 @@ __device__ void gemm_route_meta(const GemmParams& p, RouteMeta<BM>& m) {
 
 // Both: the tile, then its rows' route metadata.
 template <int BM, int NT = kGemmThreads>
-__device__ bool gemm_schedule(const GemmParams& p, int64_t tile, RouteMeta<BM>& m) {
-  if (!gemm_schedule_tile<BM>(p, tile, m)) return false;
+__device__ bool gemm_schedule(const GemmParams& p, int64_t n_groups, RouteMeta<BM>& m) {
+  if (!gemm_schedule_tile<BM>(p, n_groups, m)) return false;
   gemm_route_meta<BM, NT>(p, m);
   return true;
 }
@@ -188,12 +229,12 @@ __device__ bool gemm_schedule(const GemmParams& p, int64_t tile, RouteMeta<BM>& 
 // ceil(R / BM) + min(E, R) m-tiles has at least one surplus m-tile whenever
 // such routes exist.
 template <int BM, int NT = kGemmThreads>
-__device__ void zero_unrouted_cols(const GemmParams& p, const RouteMeta<BM>& m, int64_t tile, int64_t m_tiles,
-                                   int64_t c0, int64_t c1, int64_t dg_tile, int dg_count = 1) {
+__device__ void zero_unrouted_cols(const GemmParams& p, const RouteMeta<BM>& m, int64_t m_tiles, int64_t c0,
+                                   int64_t c1, int64_t dg_tile, int dg_count = 1) {
   const bool zero_out = p.zero_unrouted && p.out != nullptr;
   const bool zero_dg = p.dg != nullptr && dg_tile >= 0;
   if (!zero_out && !zero_dg) return;
-  const int64_t j = tile - m.row0, n_surplus = m_tiles - m.row0;
+  const int64_t j = m.tile - m.row0, n_surplus = m_tiles - m.row0;
   if (j < 0 || n_surplus <= 0) return;
   int64_t q0 = p.offsets[p.n_experts - 1];
   q0 = q0 < 0 ? 0 : q0;

@@ -46,16 +46,14 @@ __global__ __launch_bounds__(kGemmThreads, 2) void routed_gemm_kernel(const Gemm
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int64_t n_ntiles = (p.N + BN - 1) / BN;
-  const int64_t id = xcd_remap(blockIdx.x, gridDim.x);
-  const int64_t tile = id / n_ntiles;
-  const int64_t ntile = id % n_ntiles;
+  const bool tiled = gemm_schedule<BM>(p, n_ntiles, meta);
+  const int64_t ntile = uniform_i32(meta.group);
   const int64_t n0 = ntile * BN;
-
-  if (!gemm_schedule<BM>(p, tile, meta)) {
-    zero_unrouted_cols<BM>(p, meta, tile, gridDim.x / n_ntiles, n0, n0 + BN, ntile);
+  if (!tiled) {
+    zero_unrouted_cols<BM>(p, meta, gridDim.x / n_ntiles, n0, n0 + BN, ntile);
     return;
   }
-  const int32_t expert = meta.expert;
+  const int32_t expert = uniform_i32(meta.expert);
 
   OpT* As0 = reinterpret_cast<OpT*>(smem);
   OpT* Bs0 = As0 + Cfg::A_ELEMS;

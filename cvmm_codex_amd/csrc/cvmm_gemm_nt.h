@@ -68,16 +68,14 @@ __global__ __launch_bounds__(kGemmThreads, 2) void routed_gemm_nt_kernel(const G
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int64_t n_ntiles = (p.N + BN - 1) / BN;
-  const int64_t id = xcd_remap(blockIdx.x, gridDim.x);
-  const int64_t tile = id / n_ntiles;
-  const int64_t ntile = id % n_ntiles;
+  const bool tiled = gemm_schedule<BM>(p, n_ntiles, meta);
+  const int64_t ntile = uniform_i32(meta.group);
   const int64_t n0 = ntile * BN;
-
-  if (!gemm_schedule<BM>(p, tile, meta)) {
-    zero_unrouted_cols<BM>(p, meta, tile, gridDim.x / n_ntiles, n0, n0 + BN, ntile);
+  if (!tiled) {
+    zero_unrouted_cols<BM>(p, meta, gridDim.x / n_ntiles, n0, n0 + BN, ntile);
     return;
   }
-  const int32_t expert = meta.expert;
+  const int32_t expert = uniform_i32(meta.expert);
 
   // ---- per-lane DMA sources (fixed across k stages) --------------------------
   // wave instruction j covers rows 8*(wave*NA + j) .. +7; lane -> (row, physical chunk)
@@ -212,16 +210,14 @@ __global__ __launch_bounds__(kGemmThreads, 2) void routed_gemm_nloop_kernel(cons
   const int wave = tid >> 6;
   const int64_t n_ntiles = (p.N + BN - 1) / BN;
   const int64_t n_groups = (n_ntiles + ng - 1) / ng;
-  const int64_t id = xcd_remap(blockIdx.x, gridDim.x);
-  const int64_t tile = id / n_groups;
-  const int64_t nt_begin = (id % n_groups) * ng;
+  const bool tiled = gemm_schedule<BM>(p, n_groups, meta);
+  const int64_t nt_begin = uniform_i32(meta.group) * (int64_t)ng;
   const int64_t nt_end = nt_begin + ng < n_ntiles ? nt_begin + ng : n_ntiles;
-
-  if (!gemm_schedule<BM>(p, tile, meta)) {
-    zero_unrouted_cols<BM>(p, meta, tile, gridDim.x / n_groups, nt_begin * BN, nt_end * BN, -1);
+  if (!tiled) {
+    zero_unrouted_cols<BM>(p, meta, gridDim.x / n_groups, nt_begin * BN, nt_end * BN, -1);
     return;
   }
-  const int32_t expert = meta.expert;
+  const int32_t expert = uniform_i32(meta.expert);
 
   const char* zero = reinterpret_cast<const char*>(g_cvmm_zero_page);
   const char* a_src[Cfg::NA];

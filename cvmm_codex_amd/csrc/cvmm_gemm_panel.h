@@ -210,16 +210,15 @@ __global__ __launch_bounds__(kGemmThreads, (PanelCfg<KP, BN, WM>::OCC)) void rou
   const int wave = tid >> 6;
   const int64_t n_ntiles = p.N / BN;
   const int64_t n_groups = (n_ntiles + tpw - 1) / tpw;
-  const int64_t id = xcd_remap(blockIdx.x, gridDim.x);
-  const int64_t tile = id / n_groups;
-  const int64_t nt0 = (id % n_groups) * tpw;
+  const bool tiled = gemm_schedule<Cfg::BM>(p, n_groups, meta);
+  const int32_t grp = uniform_i32(meta.group);
+  const int64_t nt0 = grp * (int64_t)tpw;
   const int T = (int)((n_ntiles - nt0) < tpw ? (n_ntiles - nt0) : tpw);
-
-  if (!gemm_schedule<Cfg::BM>(p, tile, meta)) {
-    zero_unrouted_cols<Cfg::BM>(p, meta, tile, gridDim.x / n_groups, nt0 * BN, (nt0 + T) * BN, -1);
+  if (!tiled) {
+    zero_unrouted_cols<Cfg::BM>(p, meta, gridDim.x / n_groups, nt0 * BN, (nt0 + T) * BN, -1);
     return;
   }
-  const int32_t expert = meta.expert;
+  const int32_t expert = uniform_i32(meta.expert);
 
   const int wm = wave / Cfg::WN, wn = wave % Cfg::WN;
   const int fr = lane & 15, fq = lane >> 4;
@@ -352,7 +351,6 @@ __global__ __launch_bounds__(kGemmThreads, (PanelCfg<KP, BN, WM>::OCC)) void rou
   // after the first weight DMAs, so the fragment loads' wait leaves those in
   // flight; the extra stores only make the tile waits below stricter.
   if (p.xs_out != nullptr) {
-    const int64_t grp = id % n_groups;
     const int64_t G = n_groups < 4 ? n_groups : 4;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {

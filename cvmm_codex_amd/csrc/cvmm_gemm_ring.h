@@ -118,19 +118,17 @@ __global__ __launch_bounds__(NW * 64, OCC) void routed_gemm_ring_kernel(const Ge
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int64_t n_ntiles = (p.N + BN - 1) / BN;
-  const int64_t id = xcd_remap(blockIdx.x, gridDim.x);
-  const int64_t tile = id / n_ntiles;
-  const int64_t ntile = id % n_ntiles;
+  const bool tiled = gemm_schedule<BM, Cfg::NT>(p, n_ntiles, meta);
+  const int64_t ntile = uniform_i32(meta.group);
   const int64_t n0 = ntile * BN;
-
-  if (!gemm_schedule<BM, Cfg::NT>(p, tile, meta)) {
+  if (!tiled) {
     // the routing-weight gradient's partials: one per 128 columns (per tile
     // where BN = 64)
     constexpr int kDgPer = BN > 128 ? BN / 128 : 1;
-    zero_unrouted_cols<BM, Cfg::NT>(p, meta, tile, gridDim.x / n_ntiles, n0, n0 + BN, ntile * kDgPer, kDgPer);
+    zero_unrouted_cols<BM, Cfg::NT>(p, meta, gridDim.x / n_ntiles, n0, n0 + BN, ntile * kDgPer, kDgPer);
     return;
   }
-  const int32_t expert = meta.expert;
+  const int32_t expert = uniform_i32(meta.expert);
 
   // ---- per-lane DMA sources: instruction j of wave w fills LDS bytes
   // [(w * D + j) * 1024, +1024) of a slice; A rows first, then B rows ([n][k]

@@ -39,11 +39,11 @@ __global__ __launch_bounds__(256) void routed_small_kernel(const GemmParams p) {
   __shared__ RouteMeta<kSmBM> meta;
   const int tid = threadIdx.x;
   const int64_t n_ntiles = (p.N + kSmBN - 1) / kSmBN;
-  const int64_t tile = blockIdx.x / n_ntiles;
-  const int64_t n0 = (blockIdx.x % n_ntiles) * kSmBN;
   const int64_t m_tiles = gridDim.x / n_ntiles;
-  if (!gemm_schedule_tile<kSmBM>(p, tile, meta)) {
-    zero_unrouted_cols<kSmBM>(p, meta, tile, m_tiles, n0, n0 + kSmBN, -1);
+  const bool tiled = gemm_schedule_tile<kSmBM, false>(p, n_ntiles, meta);
+  const int64_t n0 = (int64_t)uniform_i32(meta.group) * kSmBN;
+  if (!tiled) {
+    zero_unrouted_cols<kSmBM>(p, meta, m_tiles, n0, n0 + kSmBN, -1);
     return;
   }
   const int64_t e = meta.expert;

@@ -1,0 +1,43 @@
+"""The routed GEMMs' tile schedule at the expert counts where its form
+changes (register-held offsets up to 256 experts, two passes beyond), with
+empty experts and ids outside the expert range, against the oracle."""
+import pytest
+import torch
+
+import cvmm_codex_amd.api as C
+from tests import gpu_util as U
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("E", [1, 64, 65, 255, 256, 257, 700])
+@pytest.mark.parametrize("D,H", [(136, 72), (64, 192)])   # long-K and small-K products
+def test_tile_schedule_over_expert_counts(E, D, H):
+    g = torch.Generator().manual_seed(E)
+    T, K = 301, 4
+    x = torch.randn(T, D, generator=g).to(torch.bfloat16)
+    keys = torch.randn(E, D, H, generator=g) / D ** 0.5
+    sel = torch.randint(0, max(1, E * 3 // 4), (T, K), generator=g)   # a quarter of the experts empty
+    sel[:, 0] = 0                                                     # one hot expert
+    go = torch.randn(T, K, H, generator=g).to(torch.bfloat16)
+    got = U.run_hip(x, keys, sel, None, go, False, True)
+    exp = U.run_oracle(x, keys, sel, None, go, False, True)
+    U.compare(got, exp, 2e-2)
+
+
+@pytest.mark.parametrize("E", [64, 257])
+def test_surplus_tiles_zero_the_unrouted_rows(E):
+    g = torch.Generator().manual_seed(E)
+    T, K, D, H = 130, 3, 136, 72
+    x = torch.randn(T, D, generator=g).to(torch.bfloat16).cuda()
+    keys = (torch.randn(E, D, H, generator=g) / D ** 0.5).cuda()
+    sel = torch.randint(0, E, (T, K), generator=g)
+    sel[torch.rand(T, K, generator=g) < 0.3] = E + 5
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = C.cvmm(x, C.cvmm_prepare_sel2(sel.cuda()), keys)
+    out_of_range = (sel >= E).cuda()
+    assert bool((y[out_of_range] == 0).all())
+    e = sel.clamp(max=E - 1).cuda()
+    ref = torch.einsum("td,tkdh->tkh", x.float(), keys.to(torch.bfloat16).float()[e])
+    err = ((y.float() - ref)[~out_of_range].abs().max() / ref.abs().max()).item()
+    assert err <= 2e-2
