@@ -52,6 +52,7 @@ _SIGS = {
     "cvmm_timing_enable": (ctypes.c_int, [ctypes.c_uint32]),
     "cvmm_tuning_set": (ctypes.c_int, [_I32, _I64]),
     "cvmm_topk_dense": (ctypes.c_int, [_I64, _I32, _I64, _I64, _I64, _I32]),
+    "cvmm_fwd_stored_keys": (ctypes.c_int, [_I64, _I32, _I64, _I64, _I32, _I32]),
     "cvmm_timing_result": (ctypes.c_int, [ctypes.c_uint32, ctypes.POINTER(ctypes.c_double),
                                           ctypes.POINTER(ctypes.c_int64)]),
     "cvmm_sort_workspace_bytes": (_SZ, [_I64, _I32]),

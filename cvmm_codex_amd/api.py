@@ -143,12 +143,23 @@ class _CopyPlan(NamedTuple):
     between the rows (kt as [d_out, E, d_in], kn as [d_in, E, d_out]: the
     GEMM's B^T rows).  Under torch.compile tracing the copies stay in the
     routed layouts and a dense sum reads the other copy as [E*K, N] rows
-    (`fwd_t` / `bwd_t` say which copy each phase reads)."""
+    (`fwd_t` / `bwd_t` say which copy each phase reads).  `stored`: kn is the
+    keys themselves, read in place (weights kept in the op dtype, or a forward
+    with few routes per expert): nothing is cast for it."""
     want_t: bool
     want_n: bool
     layout: int  # N.CAST_*_INTERLEAVED bits
     fwd_t: bool
     bwd_t: bool
+    stored: bool = False
+
+    @property
+    def cast_n(self) -> bool:
+        return self.want_n and not self.stored
+
+    @property
+    def casts(self) -> bool:
+        return self.want_t or self.cast_n
 
 
 def _sort_routes_cast(raw_flat: torch.Tensor, n_experts: int, top_k: int, cast, counted_ws=None):
@@ -157,7 +168,7 @@ def _sort_routes_cast(raw_flat: torch.Tensor, n_experts: int, top_k: int, cast, 
     CVMM.forward."""
     keys, op, plan = cast
     (ssel, perm, tok, offsets, route_pos), kt, kn = N.host().sort_routes_cast(
-        raw_flat, n_experts, top_k, keys, N.dtype_id(op), plan.want_t, plan.want_n, plan.layout,
+        raw_flat, n_experts, top_k, keys, N.dtype_id(op), plan.want_t, plan.cast_n, plan.layout,
         N.stream_of(raw_flat.device), counted_ws)
     perm._cvmm_route_pos = route_pos
     _cast_done.entry = (keys, keys._version, op, plan.layout, kt, kn)
@@ -172,9 +183,26 @@ def _take_cast(keys: torch.Tensor, op: torch.dtype, plan: _CopyPlan):
         return None
     k, version, eop, layout, kt, kn = entry
     if (k is not keys or version != keys._version or eop != op or layout != plan.layout
-            or (plan.want_t and kt is None) or (plan.want_n and kn is None)):
+            or (plan.want_t and kt is None) or (plan.cast_n and kn is None)):
         return None
     return kt, kn
+
+
+def _copies(keys: torch.Tensor, op: torch.dtype, plan: _CopyPlan):
+    """(kt, kn) of `plan`: those cast with this call's sort, or cast here; the
+    keys themselves as kn where the plan reads them in place."""
+    kt, kn = None, None
+    if plan.casts:
+        pre = None if _compiling() else _take_cast(keys, op, plan)
+        kt, kn = pre if pre is not None else _cast_keys(keys, op, plan)
+    return kt, (keys.detach() if plan.stored else kn)
+
+
+def _rows_in_place(keys: torch.Tensor) -> bool:
+    """The keys' rows of d_out values can be read 16 bytes at a time."""
+    per = 16 // keys.element_size()
+    return (keys.stride(2) == 1 and keys.stride(1) % per == 0 and keys.stride(0) % per == 0
+            and keys.data_ptr() % 16 == 0)
 
 
 @torch._dynamo.assume_constant_result
@@ -197,25 +225,36 @@ def _plan_copies(keys: torch.Tensor, op: torch.dtype, n_routes: int, top_k: int,
         fwd_t, bwd_t = not fwd_dense, bwd_dense
         return _CopyPlan(fwd_t or (need_grad_input and bwd_t), (not fwd_t) or (need_grad_input and not bwd_t),
                          0, fwd_t, bwd_t)
-    return _eager_plan(d_in, d_out, fwd_dense, bwd_dense, need_grad_input)
+    return _eager_plan(keys, op, n_routes, fwd_dense, bwd_dense, need_grad_input)
 
 
-def _eager_plan(d_in: int, d_out: int, fwd_dense: bool, bwd_dense: bool, need_grad_input: bool) -> _CopyPlan:
+def _eager_plan(keys: torch.Tensor, op: torch.dtype, n_routes: int, fwd_dense: bool, bwd_dense: bool,
+                need_grad_input: bool) -> _CopyPlan:
     """Eager copies: one copy where one product runs the long-K routed GEMM
     (K > 128), which reads the weights in either orientation, and the other
     product needs that copy's own orientation (the short-K kernel's, or a
     dense top-k sum's interleaved rows); else kt for the forward and kn for
-    the grad-input."""
+    the grad-input.  Weights kept in the op dtype are read in place of kn, and
+    a forward alone reads the weights as they are stored wherever a kernel
+    takes them so (cvmm_fwd_stored_keys): casting every expert's weights took
+    two thirds of a 32-token decode step (447 of 686 us over 128 experts of
+    2048 x 512 in bf16) and of a 1999-token prefill (449 of 768 us)."""
+    E, d_in, d_out = keys.shape
+    in_place = keys.dtype == op and _rows_in_place(keys)
     layout = (N.CAST_T_INTERLEAVED if fwd_dense else 0) | (N.CAST_N_INTERLEAVED if bwd_dense else 0)
     if not need_grad_input:
+        if (not fwd_dense and (in_place or (keys.dtype == torch.float32 and _rows_in_place(keys)))
+                and N.lib().cvmm_fwd_stored_keys(n_routes, E, d_in, d_out, _DTYPE_IDS[keys.dtype], _DTYPE_IDS[op])):
+            return _CopyPlan(False, True, 0, False, False, True)
         return _CopyPlan(True, False, layout, True, False)
     fwd_ring = d_in > 128 and not fwd_dense
     bwd_ring = d_out > 128 and not bwd_dense
+    stored = in_place and not bwd_dense
     if fwd_ring:       # kn only: the forward reads it n-contiguous
-        return _CopyPlan(False, True, layout, False, False)
+        return _CopyPlan(False, True, layout, False, False, stored)
     if bwd_ring:       # kt only: the grad-input reads it n-contiguous
         return _CopyPlan(True, False, layout, True, True)
-    return _CopyPlan(True, True, layout, True, False)
+    return _CopyPlan(True, True, layout, True, False, stored)
 
 
 def _copy_view(plan: _CopyPlan, kt, kn, fwd: bool):
@@ -680,7 +719,7 @@ def _cast_keys(keys: torch.Tensor, op: torch.dtype, plan: _CopyPlan):
     if _compiling():
         kt, kn = _ops.cast_keys(keys, op)
         return kt, kn
-    return N.host().cast_keys(keys, N.dtype_id(op), plan.want_t, plan.want_n, plan.layout,
+    return N.host().cast_keys(keys, N.dtype_id(op), plan.want_t, plan.cast_n, plan.layout,
                               N.stream_of(keys.device))
 
 
@@ -726,8 +765,7 @@ def _copies_for_call(ctx, keys, op, n_routes, top_k, weighted, token_input, need
     grad-input's kept on ctx: cast with the sort when cvmm() did that, else
     here."""
     plan = _plan_copies(keys, op, n_routes, top_k, weighted, token_input, need_grad_input)
-    pre = None if _compiling() else _take_cast(keys, op, plan)
-    kt, kn = pre if pre is not None else _cast_keys(keys, op, plan)
+    kt, kn = _copies(keys, op, plan)
     ctx.keys_x, ctx.keys_x_is_t = _copy_view(plan, kt, kn, False) if need_grad_input else (None, False)
     return _copy_view(plan, kt, kn, True)
 
@@ -825,7 +863,7 @@ def cvmm_gelu(x: torch.Tensor, sel: Union[torch.Tensor, CVMMSel], keys: torch.Te
         raw = sel._raw_shape_tensor()
         plan = _plan_copies(keys, op, raw.numel(), raw.shape[-1] if raw.ndim else 1, False,
                             not sel._route_mode, torch.is_grad_enabled() and x.requires_grad)
-        cast = (keys, op, plan)
+        cast = (keys, op, plan) if plan.casts else None
     sel._resolve(keys.shape[0], cast)
     return CVMMGelu.apply(x, sel._raw_shape_tensor(), sel.sel_index, sel.sel, keys, sel.out_index)
 
@@ -890,16 +928,15 @@ def _cvmm_eager(x: torch.Tensor, sel: Union[torch.Tensor, CVMMSel], keys: torch.
         fwd_dense = weighted and k >= 2 and not cvmm_atomic_reduce and _topk_dense(T, E, d_in, d_out, k, op_id)
         bwd_dense = (need and not weighted and token_input and k >= 2 and not cvmm_atomic_reduce
                      and _topk_dense(T, E, d_out, d_in, k, op_id))
-        plan = _eager_plan(d_in, d_out, fwd_dense, bwd_dense, need)
+        plan = _eager_plan(keys, op, raw.numel(), fwd_dense, bwd_dense, need)
     if pending:
-        sel._resolve(E, (keys, op, plan) if plan is not None else None)
+        sel._resolve(E, (keys, op, plan) if plan is not None and plan.casts else None)
     _log_shape(x, keys)
     s, sel_index, out_index = sel._sel, sel._sel_index, sel._out_index
     keys_op = keys_x = None
     fwd_t, keys_x_is_t = True, False
     if plan is not None:
-        pre = _take_cast(keys, op, plan)
-        kt, kn = pre if pre is not None else _cast_keys(keys, op, plan)
+        kt, kn = _copies(keys, op, plan)
         if need:
             keys_x, keys_x_is_t = _copy_view(plan, kt, kn, False)
         keys_op, fwd_t = _copy_view(plan, kt, kn, True)

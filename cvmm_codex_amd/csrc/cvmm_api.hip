@@ -24,6 +24,9 @@ hipError_t launch_routed_gemm_nt_bf16(const GemmParams& p, hipStream_t stream);
 hipError_t launch_routed_gemm_nt_f16(const GemmParams& p, hipStream_t stream);
 bool routed_gemm_ring_applies(const GemmParams& p, int32_t op);
 bool routed_gemm_panel_applies(const GemmParams& p, int32_t op);
+bool routed_gemm_decode_applies(const GemmParams& p, int32_t op);
+bool routed_gemm_decode_sizes(int64_t n_routes, int32_t n_experts, int64_t K, int64_t N, int32_t b_dtype);
+hipError_t launch_routed_gemm_decode(const GemmParams& p, int32_t op, hipStream_t stream);
 
 // Fast path (DMA-staged, 16-bit k-contiguous operands) when eligible, else the
 // general kernel (any storage type / stride / width).
@@ -46,8 +49,9 @@ static bool routed_gemm_is_panel(const GemmParams& p, int32_t op) {
 
 hipError_t launch_routed_gemm(const GemmParams& p, int32_t op, hipStream_t s) {
   if (small_gemm_eligible(p, op)) return launch_routed_small(p, s);
+  if (routed_gemm_decode_applies(p, op)) return launch_routed_gemm_decode(p, op, s);
   if (nt_eligible(p, op)) return op == kBF16 ? launch_routed_gemm_nt_bf16(p, s) : launch_routed_gemm_nt_f16(p, s);
-  if (p.act != 0) return hipErrorInvalidValue;  // the activation epilogue exists in the ring kernel only
+  if (p.act != 0) return hipErrorInvalidValue;  // the activation epilogue: ring and decode kernels only
   if (op == kBF16) return launch_routed_gemm_bf16(p, s);
   if (op == kF16) return launch_routed_gemm_f16(p, s);
   if (op == kF32) return launch_routed_gemm_f32(p, s);
@@ -439,6 +443,14 @@ int cvmm_tuning_set(int32_t knob, int64_t value) {
 
 int cvmm_topk_dense(int64_t n_tokens, int32_t n_experts, int64_t K, int64_t N, int64_t top_k, int32_t op_dtype) {
   return use_dense_topk(op_dtype, n_tokens, n_experts, K, N, top_k) ? 1 : 0;
+}
+
+int cvmm_fwd_stored_keys(int64_t n_routes, int32_t n_experts, int64_t d_in, int64_t d_out, int32_t keys_dtype,
+                         int32_t op_dtype) {
+  if ((op_dtype != kBF16 && op_dtype != kF16) || n_experts <= 0 || d_in <= 0 || d_out <= 0) return 0;
+  if (keys_dtype != kF32 && keys_dtype != op_dtype) return 0;
+  if (routed_gemm_decode_sizes(n_routes, n_experts, d_in, d_out, keys_dtype)) return 1;
+  return keys_dtype == op_dtype && d_in > 128 && d_in % 8 == 0 && d_out % 8 == 0 ? 1 : 0;
 }
 
 int cvmm_timing_result(uint32_t kernel_class, double* total_ms, int64_t* launches) {
@@ -859,8 +871,9 @@ static int fwd_core(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld
     p.epi = kEpiStore; p.out = out; p.out_dtype = out_dtype; p.out_ld = out_ld; p.out_rows = out_rows;
     if (pre_act != nullptr) {
       p.act = 1; p.aux = pre_act;
-      if (!(nt_eligible(p, op_dtype) && routed_gemm_ring_applies(p, op_dtype))) {
-        // not the ring kernel: the products to pre_act, then a GELU pass
+      if (!routed_gemm_decode_applies(p, op_dtype) &&
+          !(nt_eligible(p, op_dtype) && routed_gemm_ring_applies(p, op_dtype))) {
+        // a kernel without the epilogue: the products to pre_act, then a GELU pass
         p.act = 0; p.aux = nullptr; p.out = pre_act;
         int r = check_launch(timed(CVMM_KC_GEMM_FWD, s, [&] { return launch_routed_gemm(p, op_dtype, s); }), "cvmm_fwd(gemm)");
         if (r) return r;

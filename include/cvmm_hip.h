@@ -163,6 +163,15 @@ int cvmm_tuning_set(int32_t knob, int64_t value);
  * Other keys are cast into the workspace.  Returns 1 or 0. */
 int cvmm_topk_dense(int64_t n_tokens, int32_t n_experts, int64_t K, int64_t N, int64_t top_k, int32_t op_dtype);
 
+/* Whether a forward without a grad-input reads the weights best as they are
+ * stored ([E][d_in][d_out], unit stride on d_out, 16-byte aligned rows) rather
+ * than from an op-dtype copy: weights of the op dtype with a long inner
+ * dimension (d_in > 128), or few routes per expert (the kernel that streams
+ * fp32 or op-dtype weights once).  No counterpart in cvmm.py, whose kernels
+ * convert the weights per tile (cvmm.py:198-204). */
+int cvmm_fwd_stored_keys(int64_t n_routes, int32_t n_experts, int64_t d_in, int64_t d_out, int32_t keys_dtype,
+                         int32_t op_dtype);
+
 /* ------------------------------------------------------------------------ */
 /* Selector preparation                                                      */
 /* ------------------------------------------------------------------------ */
