@@ -64,7 +64,8 @@ hipError_t launch_wgrad_v3_f16(const WgradParams& p, hipStream_t stream);
 // Fast path: 16-bit x and dY in the op dtype, 16-byte aligned rows, widths % 8.
 static bool wgrad_fast_eligible(const WgradParams& p, int32_t op) {
   auto al = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-  return (op == kBF16 || op == kF16) && p.x_dtype == op && p.g_dtype == op && p.M % 8 == 0 && p.N % 8 == 0 &&
+  return (op == kBF16 || op == kF16) && p.x_dtype == op && p.g_dtype == op &&
+         (p.padded || (p.M % 8 == 0 && p.N % 8 == 0)) &&
          al(p.x) && al(p.g) && p.x_ld % 8 == 0 && p.g_ld % 8 == 0;
 }
 
@@ -373,6 +374,28 @@ int run_dense_topk(const DenseWs& w, const void* src, int32_t src_dtype, int64_t
   p.out_ld = out_ld;
   p.out_vec = aligned16(out) && (out_ld * (int64_t)dtype_size(out_dtype)) % 16 == 0;
   return check_launch(timed(gemm_class, s, [&] { return launch_topk_gemm(p, op_dtype, out_dtype, s); }), what);
+}
+
+// Widths that are not multiples of 8, 16-bit op: the operands are copied
+// into the workspace padded with zeros (cvmm_pad.hip) and the 16-byte kernels
+// run on the copies.  A training step at 412 x 130, general kernels / this,
+// GPU time of its kernels and the step with host work:
+//   32760 routes, 63 experts: 511 / 127 us, 540 / 136 us
+//    5600 routes, 64 experts: 200 / 111 us, 188 / 137 us
+//    2800 routes,  8 experts: 186 / 102 us, 172 / 169 us
+//     800 routes,  8 experts: 145 /  97 us, 145 / 162 us
+// The copies are six more launches, which the host no longer hides below
+// ~1.3e8 products: those calls keep the general kernels, and so do calls with
+// few routes per expert (16 measured: 193 / 163 us), whose weight copies
+// outweigh the products.
+bool pads_operands(int32_t op_dtype, int64_t n_routes, int32_t n_experts, int64_t d_in, int64_t d_out) {
+  if ((op_dtype != kBF16 && op_dtype != kF16) || (d_in % 8 == 0 && d_out % 8 == 0)) return false;
+  if (n_experts <= 0 || n_experts > 65535 || d_in > (1 << 20) || d_out > (1 << 20)) return false;
+  // (the copies' 16-byte pieces are counted in 31 bits)
+  const int64_t lim = 0x7fffffffll;
+  const int64_t i8 = pad8(d_in), o8 = pad8(d_out);
+  if (n_routes > lim / (i8 / 8) || n_routes > lim / (o8 / 8) || n_experts > lim / (i8 * o8 / 8)) return false;
+  return n_routes >= 16 * (int64_t)n_experts && (double)n_routes * (double)d_in * (double)d_out >= 1.34e8;
 }
 
 // n-tile width of the routed GEMM for output width n (256x64 tiles when narrow).
@@ -775,6 +798,18 @@ int cvmm_sort_routes_cast_keys_ex(const void* sel, int32_t sel_is_int64, int64_t
 }
 
 // ---------------------------------------------------------------------------
+}  // extern "C"
+
+// (an output of another type than the op's, or summed by atomics, stays with
+// the general kernels)
+static bool fwd_pads(int32_t op_dtype, int32_t out_dtype, int64_t n_routes, int32_t n_experts, int64_t d_in,
+                     int64_t d_out, int32_t flags) {
+  return out_dtype == op_dtype && !(flags & CVMM_FLAG_ATOMIC_REDUCE) &&
+         pads_operands(op_dtype, n_routes, n_experts, d_in, d_out);
+}
+
+extern "C" {
+
 size_t cvmm_fwd_workspace_bytes(int64_t n_routes, int32_t n_experts, int64_t d_in, int64_t d_out, int64_t out_rows,
                                 int32_t out_dtype, int32_t op_dtype, int32_t has_offsets, int32_t weighted,
                                 int32_t flags) {
@@ -784,13 +819,18 @@ size_t cvmm_fwd_workspace_bytes(int64_t n_routes, int32_t n_experts, int64_t d_i
                      use_dense_topk(op_dtype, out_rows, n_experts, d_in, d_out, k);
   if (dense) carve_dense(c, out_rows, n_experts, d_in, d_out, n_routes, op_dtype);
   if (!has_offsets) c.take((size_t)n_experts * 8);
+  const bool padded = fwd_pads(op_dtype, out_dtype, n_routes, n_experts, d_in, d_out, flags);
   if (weighted && !dense) {
     if (flags & CVMM_FLAG_ATOMIC_REDUCE) {
       c.take((size_t)out_rows * d_out * 4);
     } else {
-      c.take((size_t)n_routes * d_out * dtype_size(out_dtype));
+      c.take((size_t)n_routes * (padded ? pad8(d_out) : d_out) * dtype_size(out_dtype));
       c.take((size_t)n_routes * 4);
     }
+  }
+  if (padded) {
+    c.take((size_t)n_routes * pad8(d_in) * 2);
+    c.take((size_t)n_experts * pad8(d_in) * pad8(d_out) * 2);
   }
   return c.used;
 }
@@ -852,7 +892,7 @@ static int fwd_core(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld
   const int64_t bsz = (int64_t)dtype_size(keys_dtype);
   p.b_vec = aligned16(keys) && (k_se * bsz) % 16 == 0 &&
             ((k_sj == 1 && (k_si * bsz) % 16 == 0) || (k_sj != 1 && k_si == 1 && (k_sj * bsz) % 16 == 0));
-  p.K = d_in; p.N = d_out;
+  p.K = d_in; p.N = p.n_out = d_out;
   p.offsets = offs; p.n_experts = n_experts; p.n_routes = n_routes;
   const int64_t bm = routed_gemm_bm(d_out);
   p.grid_tiles = (n_routes + bm - 1) / bm + (n_experts < n_routes ? n_experts : n_routes);
@@ -863,6 +903,36 @@ static int fwd_core(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld
   p.panel_tpw = g_panel_tpw.load();
   p.ring_tile = g_ring_tile.load();
   p.token_major = gemm_token_major(n_experts);
+
+  // the route buffer of a weighted call comes before the padded copies
+  const bool pad_sizes = !dense && fwd_pads(op_dtype, out_dtype, n_routes, n_experts, d_in, d_out, flags);
+  const int64_t out_w = pad_sizes ? pad8(d_out) : d_out;
+  void* ybuf = nullptr;
+  int32_t* inv_ws = nullptr;
+  if (weighted && !dense && !(flags & CVMM_FLAG_ATOMIC_REDUCE)) {
+    ybuf = c.take((size_t)n_routes * out_w * dtype_size(out_dtype));
+    inv_ws = (int32_t*)c.take((size_t)n_routes * 4);
+  }
+  if (pad_sizes && x_rows <= n_routes) {
+    // widths off the 16-byte grid: padded copies of the rows and the weights
+    // ([k][n] rows for the long-K kernel, else [n][k])
+    const int64_t k8 = pad8(d_in), n8 = pad8(d_out);
+    void* xp = c.take((size_t)n_routes * k8 * 2);
+    void* kp = c.take((size_t)n_experts * k8 * n8 * 2);
+    int r = check_launch(timed_combine(s, [&] {
+      return launch_pad_rows(x, x_dtype, x_ld, x_rows, d_in, nullptr, 0, op_dtype, xp, s);
+    }), "cvmm_fwd(pad rows)");
+    if (r) return r;
+    const bool n_rows = k8 > 128;
+    r = check_launch(timed(CVMM_KC_CAST_KEYS, s, [&] {
+      return launch_pad_keys(keys, keys_dtype, k_se, k_si, k_sj, n_experts, d_in, d_out, op_dtype, kp, !n_rows, s);
+    }), "cvmm_fwd(pad keys)");
+    if (r) return r;
+    p.a = xp; p.a_dtype = op_dtype; p.a_ld = k8; p.a_vec = 1;
+    p.b = kp; p.b_dtype = op_dtype; p.b_vec = 1;
+    p.b_se = k8 * n8; p.b_sk = n_rows ? n8 : 1; p.b_sn = n_rows ? 1 : k8;
+    p.K = k8; p.N = n8;
+  }
 
   if (!weighted) {
     // rows of routes with an expert id outside [0, E): zeroed by the GEMM's
@@ -911,8 +981,6 @@ static int fwd_core(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld
   }
   // y in the output dtype, row q = sorted route q (contiguous rows per expert
   // tile), then the per-token combine in route order through the inverse
-  void* ybuf = c.take((size_t)n_routes * d_out * dtype_size(out_dtype));
-  int32_t* inv_ws = (int32_t*)c.take((size_t)n_routes * 4);
   const int32_t* inv = route_pos;
   int r = 0;
   if (!inv) {
@@ -920,7 +988,8 @@ static int fwd_core(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld
     if (r) return r;
     inv = inv_ws;
   }
-  p.epi = kEpiStore; p.out = ybuf; p.out_dtype = out_dtype; p.out_ld = d_out; p.out_rows = n_routes;
+  p.epi = kEpiStore; p.out = ybuf; p.out_dtype = out_dtype; p.out_ld = out_w; p.out_rows = n_routes;
+  p.n_out = p.N;  // (padded columns are products of zeros)
   p.o_idx = nullptr;
   // route input kept for the weight gradient: the small-K kernel writes the
   // scaled rows from its activation fragments (the rows cvmm_bwd_w scales)
@@ -935,7 +1004,7 @@ static int fwd_core(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld
   r = check_launch(timed(CVMM_KC_GEMM_FWD, s, [&] { return launch_routed_gemm(p, op_dtype, s); }), "cvmm_fwd(gemm)");
   if (r) return r;
   if (keep) *scaled_written = 1;
-  return check_launch(timed_combine(s, [&] { return launch_combine_rows(ybuf, out_dtype, d_out, inv, rp, offs + (n_experts - 1), rw, rw_dtype, out_dtype, out_rows, reduce_k, d_out,
+  return check_launch(timed_combine(s, [&] { return launch_combine_rows(ybuf, out_dtype, out_w, inv, rp, offs + (n_experts - 1), rw, rw_dtype, out_dtype, out_rows, reduce_k, d_out,
                                           out_dtype, out, out_dtype, out_ld, s); }),
                       "cvmm_fwd(combine)");
 }
@@ -998,6 +1067,16 @@ int cvmm_gelu_backward(const void* grad, int32_t grad_dtype, int64_t grad_ld, co
 }
 
 // ---------------------------------------------------------------------------
+}  // extern "C"
+
+static bool bwd_x_pads(int32_t op_dtype, int32_t grad_x_dtype, int64_t n_routes, int32_t n_experts, int64_t d_in,
+                       int64_t d_out, int32_t flags) {
+  return grad_x_dtype == op_dtype && !(flags & (CVMM_FLAG_ATOMIC_REDUCE | CVMM_FLAG_ACCUMULATE)) &&
+         pads_operands(op_dtype, n_routes, n_experts, d_in, d_out);
+}
+
+extern "C" {
+
 size_t cvmm_bwd_x_workspace_bytes(int64_t n_routes, int32_t n_experts, int64_t d_in, int64_t d_out,
                                   int64_t grad_x_rows, int32_t has_offsets, int32_t weighted, int32_t token_input,
                                   int64_t top_k, int32_t grad_x_dtype, int32_t op_dtype, int32_t need_grad_rw,
@@ -1009,15 +1088,21 @@ size_t cvmm_bwd_x_workspace_bytes(int64_t n_routes, int32_t n_experts, int64_t d
                      use_dense_topk(op_dtype, grad_x_rows, n_experts, d_out, d_in, top_k);
   if (dense) carve_dense(c, grad_x_rows, n_experts, d_out, d_in, n_routes, op_dtype);
   if (!has_offsets) c.take((size_t)n_experts * 8);
+  const bool padded = bwd_x_pads(op_dtype, grad_x_dtype, n_routes, n_experts, d_in, d_out, flags);
   if (reduce && !dense) {
     if (flags & CVMM_FLAG_ATOMIC_REDUCE) {
       c.take((size_t)grad_x_rows * d_in * 4);
     } else {
-      c.take((size_t)n_routes * d_in * dtype_size(weighted ? op_dtype : grad_x_dtype));
+      c.take((size_t)n_routes * (padded ? pad8(d_in) : d_in) * dtype_size(weighted ? op_dtype : grad_x_dtype));
       c.take((size_t)n_routes * 4);
     }
   }
   if (weighted && need_grad_rw) c.take((size_t)n_routes * ntiles_of(d_in, gemm_bn(d_in)) * 4);
+  if (padded) {
+    c.take((size_t)n_routes * pad8(d_out) * 2);
+    c.take((size_t)n_experts * pad8(d_in) * pad8(d_out) * 2);
+    if (weighted && need_grad_rw) c.take((size_t)n_routes * pad8(d_in) * 2);
+  }
   return c.used;
 }
 
@@ -1101,7 +1186,7 @@ int cvmm_bwd_x(const void* grad, int32_t grad_dtype, int64_t grad_rows, int64_t 
   const int64_t bsz = (int64_t)dtype_size(keys_dtype);
   p.b_vec = aligned16(keys) && (k_se * bsz) % 16 == 0 &&
             ((k_si == 1 && (k_sj * bsz) % 16 == 0) || (k_si != 1 && k_sj == 1 && (k_si * bsz) % 16 == 0));
-  p.K = d_out; p.N = d_in;
+  p.K = d_out; p.N = p.n_out = d_in;
   p.offsets = offs; p.n_experts = n_experts; p.n_routes = n_routes;
   const int64_t bm = routed_gemm_bm(d_in);
   p.grid_tiles = (n_routes + bm - 1) / bm + (n_experts < n_routes ? n_experts : n_routes);
@@ -1113,6 +1198,9 @@ int cvmm_bwd_x(const void* grad, int32_t grad_dtype, int64_t grad_rows, int64_t 
   p.ring_tile = g_ring_tile.load();
   p.token_major = gemm_token_major(n_experts);
 
+  const bool pad_sizes = bwd_x_pads(op_dtype, grad_x_dtype, n_routes, n_experts, d_in, d_out, flags);
+  const bool padded = pad_sizes && grad_rows <= n_routes && (grad_rw == nullptr || (x_rows <= n_routes && (x_dtype == kF32 || x_dtype == op_dtype)));
+  const int64_t gx_w = pad_sizes ? pad8(d_in) : d_in;
   void* route_buf = nullptr;
   const int32_t* inv = nullptr;
   float* acc = nullptr;
@@ -1136,7 +1224,7 @@ int cvmm_bwd_x(const void* grad, int32_t grad_dtype, int64_t grad_rows, int64_t 
     } else {
       // row q = sorted route q; the combine gathers each token's routes
       const int32_t bdt = weighted ? op_dtype : accumulate ? x_dtype : grad_x_dtype;
-      route_buf = c.take((size_t)n_routes * d_in * dtype_size(bdt));
+      route_buf = c.take((size_t)n_routes * gx_w * dtype_size(bdt));
       int32_t* inv_ws = (int32_t*)c.take((size_t)n_routes * 4);
       inv = route_pos;
       if (!inv) {
@@ -1145,7 +1233,7 @@ int cvmm_bwd_x(const void* grad, int32_t grad_dtype, int64_t grad_rows, int64_t 
         if (r) return r;
         inv = inv_ws;
       }
-      p.epi = kEpiStore; p.out = route_buf; p.out_dtype = bdt; p.out_ld = d_in; p.out_rows = n_routes;
+      p.epi = kEpiStore; p.out = route_buf; p.out_dtype = bdt; p.out_ld = gx_w; p.out_rows = n_routes;
       p.o_idx = nullptr;
       p.val_dtype = bdt;
     }
@@ -1165,7 +1253,38 @@ int cvmm_bwd_x(const void* grad, int32_t grad_dtype, int64_t grad_rows, int64_t 
     dg_direct = dg_nt == 1 && grad_rw_dtype == kF32;
     p.dg = dg_direct ? (float*)grad_rw : dg_part; p.dg_ntiles = (int32_t)dg_nt;
     p.dg_x = x; p.dg_x_dtype = x_dtype; p.dg_x_ld = x_ld; p.dg_x_rows = x_rows; p.dg_x_idx = sel_index;
+    p.dg_n = d_in;
     p.dg_val_dtype = op_dtype;
+  }
+
+  if (padded) {
+    // widths off the 16-byte grid: padded copies of the gradient rows, the
+    // weights (rows of d_out values) and, for the routing-weight gradient, x
+    const int64_t k8 = pad8(d_out), n8 = pad8(d_in);
+    void* gp = c.take((size_t)n_routes * k8 * 2);
+    void* kp = c.take((size_t)n_experts * k8 * n8 * 2);
+    int r = check_launch(timed_combine(s, [&] {
+      return launch_pad_rows(grad, grad_dtype, grad_ld, grad_rows, d_out, nullptr, 0, op_dtype, gp, s);
+    }), "cvmm_bwd_x(pad rows)");
+    if (r) return r;
+    r = check_launch(timed(CVMM_KC_CAST_KEYS, s, [&] {
+      return launch_pad_keys(keys, keys_dtype, k_se, k_si, k_sj, n_experts, d_in, d_out, op_dtype, kp, false, s);
+    }), "cvmm_bwd_x(pad keys)");
+    if (r) return r;
+    p.a = gp; p.a_dtype = op_dtype; p.a_ld = k8; p.a_vec = 1;
+    p.b = kp; p.b_dtype = op_dtype; p.b_vec = 1;
+    p.b_se = k8 * n8; p.b_sk = 1; p.b_sn = k8;
+    p.K = k8; p.N = n8;
+    if (route_buf != nullptr) p.n_out = n8;  // (padded columns are products of zeros)
+    // (fp32 x stays as it is: its unrounded values enter the gradient)
+    if (weighted && grad_rw && x_dtype == op_dtype) {
+      void* xp = c.take((size_t)n_routes * n8 * 2);
+      r = check_launch(timed_combine(s, [&] {
+        return launch_pad_rows(x, x_dtype, x_ld, x_rows, d_in, nullptr, 0, op_dtype, xp, s);
+      }), "cvmm_bwd_x(pad x)");
+      if (r) return r;
+      p.dg_x = xp; p.dg_x_ld = p.dg_n = n8;
+    }
   }
 
   int r = check_launch(timed(CVMM_KC_GEMM_BWDX, s, [&] { return launch_routed_gemm(p, op_dtype, s); }), "cvmm_bwd_x(gemm)");
@@ -1177,7 +1296,7 @@ int cvmm_bwd_x(const void* grad, int32_t grad_dtype, int64_t grad_rows, int64_t 
                        "cvmm_bwd_x(cast)");
     } else {
       const int32_t bdt = weighted ? op_dtype : accumulate ? x_dtype : grad_x_dtype;
-      r = check_launch(timed_combine(s, [&] { return launch_combine_rows(route_buf, bdt, d_in, inv, rp, offs + (n_experts - 1), weighted ? rw : nullptr, rw_dtype, op_dtype,
+      r = check_launch(timed_combine(s, [&] { return launch_combine_rows(route_buf, bdt, gx_w, inv, rp, offs + (n_experts - 1), weighted ? rw : nullptr, rw_dtype, op_dtype,
                                            grad_x_rows, top_k, d_in, weighted ? op_dtype : -1, grad_x, grad_x_dtype,
                                            grad_x_ld, s, accumulate); }),
                        "cvmm_bwd_x(combine)");
@@ -1226,6 +1345,8 @@ size_t cvmm_bwd_w_workspace_bytes(int64_t n_routes, int32_t n_experts, int64_t d
 size_t cvmm_bwd_w_workspace_bytes_ex(int64_t n_routes, int32_t n_experts, int64_t d_in, int64_t d_out,
                                      int32_t op_dtype, int32_t has_offsets, int32_t weighted_route_input) {
   size_t need = cvmm_bwd_w_workspace_bytes(n_routes, n_experts, d_in, d_out, op_dtype, has_offsets);
+  if (pads_operands(op_dtype, n_routes, n_experts, d_in, d_out))  // padded x and gradient rows
+    return align_up(need, 256) + align_up((size_t)n_routes * pad8(d_in) * 2, 256) + (size_t)n_routes * pad8(d_out) * 2;
   if (weighted_route_input && wgrad_scales_rows(op_dtype, d_in))
     need = align_up(need, 256) + (size_t)n_routes * d_in * dtype_size(op_dtype);
   return need;
@@ -1293,9 +1414,31 @@ int cvmm_bwd_w(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld, con
   // (the weight moves from the d_out-wide gradient slices of every dW tile to
   // one pass over the d_in-wide route rows).
   const size_t rows_bytes = (size_t)x_rows * d_in * dtype_size(op_dtype);
-  const bool scale_rows = !rows_scaled && weighted && out_index == nullptr && x_rows <= n_routes && n_routes > 0 &&
+  // Widths off the 16-byte grid, where the workspace holds the padded copies
+  // (the x rows of a weighted route-input selection scaled on the way).
+  const bool padded = pads_operands(op_dtype, n_routes, n_experts, d_in, d_out) && !rows_scaled && x_rows <= n_routes &&
+                      grad_rows <= n_routes &&
+                      align_up(c.used, 256) + align_up((size_t)n_routes * pad8(d_in) * 2, 256) +
+                              (size_t)n_routes * pad8(d_out) * 2 <= workspace_bytes;
+  const bool scale_rows = !padded && !rows_scaled && weighted && out_index == nullptr && x_rows <= n_routes && n_routes > 0 &&
                           wgrad_scales_rows(op_dtype, d_in) && align_up(c.used, 256) + rows_bytes <= workspace_bytes;
-  if (rows_scaled) {
+  if (padded) {
+    const bool scaled = weighted && out_index == nullptr;
+    void* xp = c.take((size_t)n_routes * pad8(d_in) * 2);
+    void* gp = c.take((size_t)n_routes * pad8(d_out) * 2);
+    int r = check_launch(timed_combine(s, [&] {
+      return launch_pad_rows(x, x_dtype, x_ld, x_rows, d_in, scaled ? rw : nullptr, rw_dtype, op_dtype, xp, s);
+    }), "cvmm_bwd_w(pad x)");
+    if (r) return r;
+    r = check_launch(timed_combine(s, [&] {
+      return launch_pad_rows(grad, grad_dtype, grad_ld, grad_rows, d_out, nullptr, 0, op_dtype, gp, s);
+    }), "cvmm_bwd_w(pad grad)");
+    if (r) return r;
+    x = xp; x_dtype = op_dtype; x_ld = pad8(d_in);
+    grad = gp; grad_dtype = op_dtype; grad_ld = pad8(d_out);
+    if (scaled) rw = nullptr;
+    p.padded = 1;
+  } else if (rows_scaled) {
     rw = nullptr;  // (the selection stays weighted: one gradient row per token)
   } else if (scale_rows) {
     void* xs = c.take(rows_bytes);

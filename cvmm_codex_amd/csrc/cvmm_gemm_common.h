@@ -217,6 +217,25 @@ __device__ bool gemm_schedule(const GemmParams& p, int64_t n_groups, RouteMeta<B
   return true;
 }
 
+// 16 bytes of a row (4 / 2-byte elements, `left` of them inside the row) at
+// any element alignment: one store where they all are.
+template <int ESZ>
+__device__ __forceinline__ void store_piece(char* dst, const uint32_t (&d)[4], int64_t left) {
+  if (left >= 16 / ESZ) {
+    __builtin_memcpy(dst, d, 16);
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (left >= (i + 1) * (4 / ESZ)) {
+      __builtin_memcpy(dst + 4 * i, &d[i], 4);
+    } else if (ESZ == 2 && left == 2 * i + 1) {
+      const uint16_t h = (uint16_t)d[i];
+      __builtin_memcpy(dst + 4 * i, &h, 2);
+    }
+  }
+}
+
 // Called by a workgroup past the last m-tile (gemm_schedule returned false,
 // leaving the tile count in m.row0), for the routes no tile covers -- expert
 // id outside [0, E), sorted at or past offsets[E - 1]: when the call asks
@@ -238,7 +257,7 @@ __device__ void zero_unrouted_cols(const GemmParams& p, const RouteMeta<BM>& m, 
   if (j < 0 || n_surplus <= 0) return;
   int64_t q0 = p.offsets[p.n_experts - 1];
   q0 = q0 < 0 ? 0 : q0;
-  if (c1 > p.N) c1 = p.N;
+  if (c1 > p.n_out) c1 = p.n_out;
   for (int64_t q = q0 + j; q < p.n_routes; q += n_surplus) {
     if (zero_dg && threadIdx.x == 0) {
       const int64_t wi = p.w_idx[q];
@@ -289,7 +308,7 @@ __device__ void gemm_epilogue(const GemmParams& p, const float* C0, const float*
       }
       const int64_t nb = n0 + cg * 8;
       const int64_t off = orow * p.out_ld + nb;
-      if (ovec && nb + 8 <= p.N) {
+      if (ovec && nb + 8 <= p.n_out) {
         Chunk16 ch;
         if (p.out_dtype == kBF16) {
 #pragma unroll
@@ -302,14 +321,14 @@ __device__ void gemm_epilogue(const GemmParams& p, const float* C0, const float*
       } else {
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-          if (nb + j < p.N) store_from_f32(p.out, p.out_dtype, off + j, v[j]);
+          if (nb + j < p.n_out) store_from_f32(p.out, p.out_dtype, off + j, v[j]);
       }
     }
   } else {  // kEpiAtomic: consecutive lanes -> consecutive columns of one row
     float* out = reinterpret_cast<float*>(p.out);
     const int col = tid % BN;
     const int64_t n = n0 + col;
-    if (n < p.N) {
+    if (n < p.n_out) {
       for (int r = tid / BN; r < rows; r += kGemmThreads / BN) {
         const int64_t orow = m.orow[r];
         if (orow < 0) continue;
@@ -335,7 +354,7 @@ __device__ void gemm_epilogue(const GemmParams& p, const float* C0, const float*
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const int64_t n = n0 + cg * 8 + j;
-          if (n < p.N)
+          if (n < p.dg_n)
             s += round_to(crow(r)[cg * 8 + j], p.dg_val_dtype) *
                  load_as_f32(p.dg_x, p.dg_x_dtype, xr * p.dg_x_ld + n);
         }

@@ -203,7 +203,7 @@ inline bool decode_eligible(const GemmParams& p, int32_t op) {
   return (op == kBF16 || op == kF16) && p.role == 0 && decode_sizes_ok(p.n_routes, p.n_experts, p.K, p.N, p.b_dtype) &&
          p.a_dtype == op && (p.b_dtype == op || p.b_dtype == kF32) && p.out_dtype == op && p.val_dtype == op &&
          p.b_sn == 1 && p.b_sk % bv == 0 && p.b_se % bv == 0 && p.a_ld % 8 == 0 && p.out_ld % 8 == 0 && al(p.a) &&
-         al(p.b) && al(p.out) && p.epi == kEpiStore && p.out != nullptr && p.w == nullptr && p.dg == nullptr &&
+         al(p.b) && al(p.out) && p.n_out == p.N && p.epi == kEpiStore && p.out != nullptr && p.w == nullptr && p.dg == nullptr &&
          p.xs_out == nullptr && (p.act == 0 || (p.aux != nullptr && al(p.aux)));
 }
 

@@ -410,7 +410,7 @@ hipError_t launch_routed_gemm_nt_op(const GemmParams& p, hipStream_t stream) {
   const int64_t nk = (p.K + 63) / 64;
   const int64_t n_ntiles = (p.N + 127) / 128;
   if (nk == 1 && n_ntiles > 1 && p.epi == kEpiStore && p.dg == nullptr && p.out != nullptr && p.N % 8 == 0 &&
-      p.out_ld % 8 == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0)
+      p.n_out == p.N && p.out_ld % 8 == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0)
     return launch_routed_gemm_nloop_t<OpT, 128, 128>(p, (int32_t)n_ntiles, stream);
   return launch_routed_gemm_nt_t<OpT, 128, 128>(p, stream);
 }

@@ -358,8 +358,11 @@ __global__ __launch_bounds__(NW * 64, OCC) void routed_gemm_ring_kernel(const Ge
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int64_t n = nwave + i * 16 + 4 * fq;
-        if (rowp != nullptr && n < p.N)
-          *reinterpret_cast<float4*>(rowp + n * 4) = make_float4(v[i][0], v[i][1], v[i][2], v[i][3]);
+        if (rowp != nullptr && n < p.n_out) {
+          const uint32_t d[4] = {__float_as_uint(v[i][0]), __float_as_uint(v[i][1]), __float_as_uint(v[i][2]),
+                                 __float_as_uint(v[i][3])};
+          store_piece<4>(rowp + n * 4, d, p.n_out - n);
+        }
       }
     } else {
       // blocks 2p, 2p+1 -> columns 32p + 8*fq + [0, 8) per lane (two lane swaps)
@@ -381,8 +384,10 @@ __global__ __launch_bounds__(NW * 64, OCC) void routed_gemm_ring_kernel(const Ge
         const auto t0 = __builtin_amdgcn_permlane16_swap(s0[0], s0[1], false, false);
         const auto t1 = __builtin_amdgcn_permlane16_swap(s1[0], s1[1], false, false);
         const int64_t n = nwave + pr * 32 + 8 * fq;
-        if (rowp != nullptr && n < p.N)
-          *reinterpret_cast<uint4*>(rowp + n * 2) = make_uint4(t0[0], t1[0], t0[1], t1[1]);
+        if (rowp != nullptr && n < p.n_out) {
+          const uint32_t d[4] = {t0[0], t1[0], t0[1], t1[1]};
+          store_piece<2>(rowp + n * 2, d, p.n_out - n);
+        }
       }
     }
   };
@@ -499,7 +504,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void routed_gemm_ring_kernel(const Ge
 // routing weight, optionally with the routing-weight gradient partials of
 // its n tile, of gemm_bn(N) columns, against 16-bit x with 8-byte aligned
 // rows), output in the op type or fp32, N a multiple of 8 with 16-byte
-// aligned output rows.
+// aligned output rows (any rows where N counts padding).
 inline bool ring_eligible(const GemmParams& p, int32_t op) {
   const size_t esz = p.out_dtype == kF32 ? 4 : 2;
   // weights k-contiguous, or n-contiguous with 16-byte aligned k rows
@@ -509,9 +514,10 @@ inline bool ring_eligible(const GemmParams& p, int32_t op) {
          (p.dg == nullptr || (p.act == 0 && p.dg_ntiles == (p.N + (p.N <= 64 ? 63 : 127)) / (p.N <= 64 ? 64 : 128) &&
                               (p.dg_x_dtype == kBF16 || p.dg_x_dtype == kF16) &&
                               (reinterpret_cast<uintptr_t>(p.dg_x) & 7) == 0 && p.dg_x_ld % 4 == 0)) &&
-         (p.act == 0 || (p.aux != nullptr && (reinterpret_cast<uintptr_t>(p.aux) % 16) == 0)) &&
+         (p.act == 0 || (p.aux != nullptr && (p.n_out < p.N || (reinterpret_cast<uintptr_t>(p.aux) % 16) == 0))) &&
          (p.out_dtype == op || p.out_dtype == kF32) && p.N % 8 == 0 &&
-         (reinterpret_cast<uintptr_t>(p.out) % 16) == 0 && ((size_t)p.out_ld * esz) % 16 == 0;
+         // (a padded N stores rows of n_out columns at any alignment)
+         (p.n_out < p.N || ((reinterpret_cast<uintptr_t>(p.out) % 16) == 0 && ((size_t)p.out_ld * esz) % 16 == 0));
 }
 
 template <typename OpT, typename OutT, int BM, int BN, int STAGES, int OCC, bool RA, int BK, bool BNC, int NW>

@@ -11,6 +11,7 @@
 namespace cvmm {
 
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
+inline int64_t pad8(int64_t n) { return (n + 7) / 8 * 8; }
 
 // ---------------------------------------------------------------------------
 // routed GEMM:  for every expert-sorted route p,
@@ -37,6 +38,7 @@ struct GemmParams {
   int64_t b_se, b_sk, b_sn;
   int32_t b_vec;
   int64_t K, N;
+  int64_t n_out;           // columns stored: N, or fewer where N counts zero padding up to a multiple of 8
   // route grouping
   const int64_t* offsets;  // inclusive per-expert offsets, int64[E]
   int32_t n_experts;
@@ -62,6 +64,7 @@ struct GemmParams {
   const void* dg_x;
   int32_t dg_x_dtype;
   int64_t dg_x_ld, dg_x_rows;
+  int64_t dg_n;            // columns of dg_x (N, or fewer where N counts zero padding and dg_x is not padded)
   const int64_t* dg_x_idx;
   int32_t dg_val_dtype;
   // 0 = forward, 1 = grad-input: selects separately named kernel
@@ -133,6 +136,7 @@ struct WgradParams {
   int64_t max_slots;
   int32_t* counters;       // [E][tiles_m*tiles_n], zero on entry
   int32_t order;           // workgroup order, one of kWgOrder*
+  int32_t padded;          // x and g rows hold zeros up to a multiple of 8 columns past M and N
   int32_t tile_choice;     // 16-bit fast path tile: kWgTile*
 };
 
@@ -267,6 +271,15 @@ hipError_t launch_route_topk_backward(const void* logits, int32_t logits_dtype, 
                                       int32_t n_experts, int64_t top_k, int32_t renormalize, const int64_t* sel,
                                       const float* grad_weights, void* grad_logits, int64_t grad_ld,
                                       hipStream_t stream);
+
+// Op-dtype copies padded with zeros to multiples of 8 (cvmm_pad.hip): rows
+// (with w: scaled by their rounded weight, one per row), and the expert
+// matrices keys[e][i][j] as [E][i8][j8] or, transposed, [E][j8][i8].
+hipError_t launch_pad_rows(const void* src, int32_t src_dtype, int64_t ld, int64_t rows, int64_t n, const void* w,
+                           int32_t w_dtype, int32_t op_dtype, void* dst, hipStream_t stream);
+hipError_t launch_pad_keys(const void* keys, int32_t keys_dtype, int64_t se, int64_t si, int64_t sj,
+                           int32_t n_experts, int64_t d_i, int64_t d_j, int32_t op_dtype, void* dst,
+                           bool transposed, hipStream_t stream);
 
 hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t stream);
 // out[i] = (int32) sel[i] (int64 ids: their low 32 bits)

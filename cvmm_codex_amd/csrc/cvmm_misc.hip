@@ -70,17 +70,15 @@ hipError_t launch_copy_ids(const void* sel, bool sel_is_int64, int64_t n, int32_
   return hipGetLastError();
 }
 
-// 8 consecutive columns of any storage type as floats (vector when aligned).
-__device__ __forceinline__ void load8_any(const void* p, int32_t dt, int64_t off, bool vec, int64_t nvalid,
-                                          float (&v)[8]) {
-  if (vec && nvalid >= 8) {
+// 8 consecutive columns of any storage type as floats: one or two 16-byte
+// accesses at any element alignment, element by element at a row's end.
+__device__ __forceinline__ void load8_any(const void* p, int32_t dt, int64_t off, int64_t nvalid, float (&v)[8]) {
+  if (nvalid >= 8) {
     if (dt == kF32) {
-      const float4 a = *reinterpret_cast<const float4*>((const float*)p + off);
-      const float4 b = *reinterpret_cast<const float4*>((const float*)p + off + 4);
-      v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+      __builtin_memcpy(v, (const float*)p + off, 32);
     } else {
       Chunk16 c;
-      c.u = *reinterpret_cast<const uint4*>((const uint16_t*)p + off);
+      __builtin_memcpy(&c, (const uint16_t*)p + off, 16);
       if (dt == kBF16) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = (float)c.b[j];
@@ -95,12 +93,10 @@ __device__ __forceinline__ void load8_any(const void* p, int32_t dt, int64_t off
   }
 }
 
-__device__ __forceinline__ void store8_any(void* p, int32_t dt, int64_t off, bool vec, int64_t nvalid,
-                                           const float (&v)[8]) {
-  if (vec && nvalid >= 8) {
+__device__ __forceinline__ void store8_any(void* p, int32_t dt, int64_t off, int64_t nvalid, const float (&v)[8]) {
+  if (nvalid >= 8) {
     if (dt == kF32) {
-      *reinterpret_cast<float4*>((float*)p + off) = make_float4(v[0], v[1], v[2], v[3]);
-      *reinterpret_cast<float4*>((float*)p + off + 4) = make_float4(v[4], v[5], v[6], v[7]);
+      __builtin_memcpy((float*)p + off, v, 32);
     } else {
       Chunk16 c;
       if (dt == kBF16) {
@@ -110,7 +106,7 @@ __device__ __forceinline__ void store8_any(void* p, int32_t dt, int64_t off, boo
 #pragma unroll
         for (int j = 0; j < 8; ++j) c.h[j] = (f16_t)v[j];
       }
-      *reinterpret_cast<uint4*>((uint16_t*)p + off) = c.u;
+      __builtin_memcpy((uint16_t*)p + off, &c, 16);
     }
   } else {
 #pragma unroll
@@ -132,7 +128,7 @@ __global__ __launch_bounds__(256) void combine_rows_kernel(
     const void* __restrict__ buf, int32_t buf_dtype, int64_t buf_ld, const int32_t* __restrict__ inv,
     const int64_t* __restrict__ rp, int64_t n_routes, const int64_t* __restrict__ rows_end, const void* __restrict__ w,
     int32_t w_dtype, int32_t w_round, int64_t k, int64_t n, int32_t mid_dtype, void* __restrict__ out,
-    int32_t out_dtype, int64_t out_ld, bool in_vec, bool out_vec) {
+    int32_t out_dtype, int64_t out_ld) {
   // the token's routes are resolved once per workgroup (64 at a time) into
   // LDS: row of the route in `buf` (-1: none) and its rounded weight
   __shared__ int64_t s_row[64];
@@ -162,7 +158,7 @@ __global__ __launch_bounds__(256) void combine_rows_kernel(
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int64_t row = s_row[j + u];
-          if (row >= 0) load8_any(buf, buf_dtype, row * buf_ld + c, in_vec, n - c, v[u]);
+          if (row >= 0) load8_any(buf, buf_dtype, row * buf_ld + c, n - c, v[u]);
           else {
 #pragma unroll
             for (int q = 0; q < 8; ++q) v[u][q] = 0.f;
@@ -179,7 +175,7 @@ __global__ __launch_bounds__(256) void combine_rows_kernel(
         const int64_t row = s_row[j];
         if (row < 0) continue;
         float v[8];
-        load8_any(buf, buf_dtype, row * buf_ld + c, in_vec, n - c, v);
+        load8_any(buf, buf_dtype, row * buf_ld + c, n - c, v);
         const float wv = s_w[j];
 #pragma unroll
         for (int q = 0; q < 8; ++q) acc[q] += wv * v[q];
@@ -192,7 +188,7 @@ __global__ __launch_bounds__(256) void combine_rows_kernel(
 #pragma unroll
     for (int q = 0; q < 8; ++q) acc[q] = round_to(acc[q], mid_dtype);
   }
-  store8_any(out, out_dtype, t * out_ld + c, out_vec, n - c, acc);
+  store8_any(out, out_dtype, t * out_ld + c, n - c, acc);
 }
 
 // The same sum with one wave per token, for 16-bit row buffers with aligned
@@ -276,7 +272,7 @@ __global__ __launch_bounds__(256) void combine_rows_wave_kernel(
         for (int q = 0; q < 8; ++q) acc[pc][q] = round_to(acc[pc][q], mid_dtype);
       }
       const int64_t c = cb + pc * 512 + lane * 8;
-      if (in[pc]) store8_any(out, out_dtype, t * out_ld + c, true, n - c, acc[pc]);
+      if (in[pc]) store8_any(out, out_dtype, t * out_ld + c, n - c, acc[pc]);
     }
   }
 }
@@ -314,10 +310,12 @@ hipError_t launch_combine_rows(const void* buf, int32_t buf_dtype, int64_t buf_l
   if (n_tokens <= 0 || n <= 0) return hipSuccess;
   if (n_tokens > 0x7fffffffll || (n + 2047) / 2048 > 65535) return hipErrorInvalidValue;
   if ((inv == nullptr) != (rp == nullptr)) return hipErrorInvalidValue;
-  const bool wave_ok = (buf_dtype == kBF16 || buf_dtype == kF16) && k <= 64 && n % 8 == 0 &&
-                       vec_ok(buf, buf_dtype, buf_ld) && vec_ok(out, out_dtype, out_ld);
+  // (buffer rows of whole 16-byte pieces, padded past n where n is no
+  // multiple of 8; output rows at any alignment)
+  const bool wave_ok = (buf_dtype == kBF16 || buf_dtype == kF16) && k <= 64 && buf_ld >= pad8(n) &&
+                       vec_ok(buf, buf_dtype, buf_ld);
   // a running sum: fp32 rows, added to unrounded, by the wave kernel only
-  if (accumulate && !(wave_ok && out_dtype == kF32 && mid_dtype < 0)) return hipErrorInvalidValue;
+  if (accumulate && !(wave_ok && n % 8 == 0 && vec_ok(out, out_dtype, out_ld) && out_dtype == kF32 && mid_dtype < 0)) return hipErrorInvalidValue;
   if (wave_ok) {
     const dim3 grid((unsigned)((n_tokens + 3) / 4));
     // whole 2048-column rows per batch where rows are that wide; 1024 columns
@@ -340,24 +338,22 @@ hipError_t launch_combine_rows(const void* buf, int32_t buf_dtype, int64_t buf_l
   dim3 grid, block;
   rows_grid(n_tokens, n, &grid, &block);
   hipLaunchKernelGGL(combine_rows_kernel, grid, block, 0, stream, buf, buf_dtype, buf_ld, inv, rp, n_tokens * k,
-                     rows_end, w, w_dtype, w_round, k, n, mid_dtype, out, out_dtype, out_ld, vec_ok(buf, buf_dtype, buf_ld),
-                     vec_ok(out, out_dtype, out_ld));
+                     rows_end, w, w_dtype, w_round, k, n, mid_dtype, out, out_dtype, out_ld);
   return hipGetLastError();
 }
 
 __global__ void cast_rows_kernel(const float* __restrict__ acc, int64_t acc_ld, int64_t n, int32_t mid_dtype,
-                                 void* __restrict__ out, int32_t out_dtype, int64_t out_ld, bool in_vec,
-                                 bool out_vec) {
+                                 void* __restrict__ out, int32_t out_dtype, int64_t out_ld) {
   const int64_t t = blockIdx.x;
   const int64_t c = ((int64_t)blockIdx.y * blockDim.x + threadIdx.x) * 8;
   if (c >= n) return;
   float v[8];
-  load8_any(acc, kF32, t * acc_ld + c, in_vec, n - c, v);
+  load8_any(acc, kF32, t * acc_ld + c, n - c, v);
   if (mid_dtype >= 0) {
 #pragma unroll
     for (int q = 0; q < 8; ++q) v[q] = round_to(v[q], mid_dtype);
   }
-  store8_any(out, out_dtype, t * out_ld + c, out_vec, n - c, v);
+  store8_any(out, out_dtype, t * out_ld + c, n - c, v);
 }
 
 hipError_t launch_cast_rows(const float* acc, int64_t acc_ld, int64_t rows, int64_t n, int32_t mid_dtype,
@@ -366,8 +362,7 @@ hipError_t launch_cast_rows(const float* acc, int64_t acc_ld, int64_t rows, int6
   if (rows > 0x7fffffffll || (n + 2047) / 2048 > 65535) return hipErrorInvalidValue;
   dim3 grid, block;
   rows_grid(rows, n, &grid, &block);
-  hipLaunchKernelGGL(cast_rows_kernel, grid, block, 0, stream, acc, acc_ld, n, mid_dtype, out, out_dtype, out_ld,
-                     vec_ok(acc, kF32, acc_ld), vec_ok(out, out_dtype, out_ld));
+  hipLaunchKernelGGL(cast_rows_kernel, grid, block, 0, stream, acc, acc_ld, n, mid_dtype, out, out_dtype, out_ld);
   return hipGetLastError();
 }
 
@@ -411,7 +406,7 @@ __device__ __forceinline__ void gelu_piece(int64_t i, int64_t cols8, bool flat, 
 // y = rnd(gelu(h)) per element (F.gelu, erf form).
 __global__ __launch_bounds__(256) void gelu_rows_kernel(const void* __restrict__ h, int32_t h_dtype, int64_t h_ld,
                                                         int64_t rows, int64_t cols, void* __restrict__ y,
-                                                        int32_t y_dtype, int64_t y_ld, bool in_vec, bool out_vec,
+                                                        int32_t y_dtype, int64_t y_ld,
                                                         bool flat) {
   const int64_t cols8 = (cols + 7) / 8;
   const int64_t n = rows * cols8;
@@ -420,18 +415,17 @@ __global__ __launch_bounds__(256) void gelu_rows_kernel(const void* __restrict__
     int64_t r, c;
     gelu_piece(i, cols8, flat, &r, &c);
     float v[8];
-    load8_any(h, h_dtype, r * h_ld + c, in_vec, lim - c, v);
+    load8_any(h, h_dtype, r * h_ld + c, lim - c, v);
 #pragma unroll
     for (int q = 0; q < 8; ++q) v[q] = gelu_erf(v[q]);
-    store8_any(y, y_dtype, r * y_ld + c, out_vec, lim - c, v);
+    store8_any(y, y_dtype, r * y_ld + c, lim - c, v);
   }
 }
 
 // dh = rnd(dy * gelu'(h)) per element (the gelu backward formula).
 __global__ __launch_bounds__(256) void gelu_backward_kernel(
     const void* __restrict__ dy, int32_t dy_dtype, int64_t dy_ld, const void* __restrict__ h, int32_t h_dtype,
-    int64_t h_ld, int64_t rows, int64_t cols, void* __restrict__ dh, int32_t dh_dtype, int64_t dh_ld, bool dy_vec,
-    bool h_vec, bool out_vec, bool flat) {
+    int64_t h_ld, int64_t rows, int64_t cols, void* __restrict__ dh, int32_t dh_dtype, int64_t dh_ld, bool flat) {
   const int64_t cols8 = (cols + 7) / 8;
   const int64_t n = rows * cols8;
   const int64_t lim = flat ? rows * cols : cols;
@@ -439,11 +433,11 @@ __global__ __launch_bounds__(256) void gelu_backward_kernel(
     int64_t r, c;
     gelu_piece(i, cols8, flat, &r, &c);
     float g[8], x[8];
-    load8_any(dy, dy_dtype, r * dy_ld + c, dy_vec, lim - c, g);
-    load8_any(h, h_dtype, r * h_ld + c, h_vec, lim - c, x);
+    load8_any(dy, dy_dtype, r * dy_ld + c, lim - c, g);
+    load8_any(h, h_dtype, r * h_ld + c, lim - c, x);
 #pragma unroll
     for (int q = 0; q < 8; ++q) g[q] = g[q] * gelu_erf_grad(x[q]);
-    store8_any(dh, dh_dtype, r * dh_ld + c, out_vec, lim - c, g);
+    store8_any(dh, dh_dtype, r * dh_ld + c, lim - c, g);
   }
 }
 
@@ -490,7 +484,7 @@ hipError_t launch_gelu_rows(const void* h, int32_t h_dtype, int64_t h_ld, int64_
   if (rows <= 0 || cols <= 0) return hipSuccess;
   if (rows * ((cols + 7) / 8) > 0xffffffffll) return hipErrorInvalidValue;  // 32-bit row split
   hipLaunchKernelGGL(gelu_rows_kernel, dim3(gelu_grid(rows, cols)), dim3(256), 0, stream, h, h_dtype, h_ld, rows,
-                     cols, y, y_dtype, y_ld, vec_ok(h, h_dtype, h_ld), vec_ok(y, y_dtype, y_ld),
+                     cols, y, y_dtype, y_ld,
                      gelu_flat(cols, h_ld, y_ld, cols));
   return hipGetLastError();
 }
@@ -514,8 +508,7 @@ hipError_t launch_gelu_backward(const void* dy, int32_t dy_dtype, int64_t dy_ld,
     return hipGetLastError();
   }
   hipLaunchKernelGGL(gelu_backward_kernel, dim3(gelu_grid(rows, cols)), dim3(256), 0, stream, dy, dy_dtype, dy_ld, h,
-                     h_dtype, h_ld, rows, cols, dh, dh_dtype, dh_ld, vec_ok(dy, dy_dtype, dy_ld),
-                     vec_ok(h, h_dtype, h_ld), vec_ok(dh, dh_dtype, dh_ld), gelu_flat(cols, dy_ld, h_ld, dh_ld));
+                     h_dtype, h_ld, rows, cols, dh, dh_dtype, dh_ld, gelu_flat(cols, dy_ld, h_ld, dh_ld));
   return hipGetLastError();
 }
 

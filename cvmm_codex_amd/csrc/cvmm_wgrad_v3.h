@@ -130,10 +130,18 @@ __device__ __forceinline__ bool wgrad_schedule(const WgradParams& p, int64_t slo
   return s.expert >= 0;
 }
 
-// dW contiguous fp32 rows, 16-byte aligned: a lane's 4 columns are one store.
-__host__ __device__ inline bool wgrad_dw_vec(const WgradParams& p) {
-  return p.dw_sn == 1 && p.dw_dtype == kF32 && p.dw_sm % 4 == 0 && p.dw_se % 4 == 0 &&
-         (reinterpret_cast<uintptr_t>(p.dw) & 15) == 0;
+// dW of fp32 rows: a lane's 4 columns are one store (at any alignment; the
+// row's last piece may be shorter).
+__host__ __device__ inline bool wgrad_dw_vec(const WgradParams& p) { return p.dw_sn == 1 && p.dw_dtype == kF32; }
+
+__device__ __forceinline__ void wgrad_store4(float* row, int64_t n, int64_t N, const float4& v) {
+  if (n + 4 <= N) {
+    __builtin_memcpy(row + n, &v, 16);
+  } else {
+    row[n] = v.x;
+    if (n + 1 < N) row[n + 1] = v.y;
+    if (n + 2 < N) row[n + 2] = v.z;
+  }
 }
 
 template <typename OpT, int BM, int BN, int WM, int WN, int STAGES, bool WEIGHTED>
@@ -334,8 +342,8 @@ __global__ __launch_bounds__(WM * WN * 64, (BM / WM / 16) * (BN / WN / 16) <= 16
   vm_wait<0>();
 
   // ---- epilogue: lane holds dW[m = m0 + wm*16*JM + j*16 + L][n = n0 + wn*16*IN + i*16 + 4*grp + {0..3}]
-  // one-workgroup-per-CU tiles are launched only for contiguous, aligned
-  // fp32 dW (wgrad_dw_vec): their accumulators never take the element path
+  // one-workgroup-per-CU tiles are launched only for fp32 dW with unit
+  // column stride (wgrad_dw_vec): their accumulators never take the element path
   constexpr bool VEC_ONLY = Cfg::OCC == 1;
   const bool dw_vec = VEC_ONLY || wgrad_dw_vec(p);
   // Stores are emitted per 16 x 16 block straight from where the block's sum
@@ -351,7 +359,7 @@ __global__ __launch_bounds__(WM * WN * 64, (BM / WM / 16) * (BN / WN / 16) <= 16
 #pragma unroll
         for (int i = 0; i < IN; ++i) {
           const int64_t n = n0 + wn * 16 * IN + i * 16 + 4 * grp;
-          if (n < p.N) *reinterpret_cast<float4*>(row + n) = block(i, j);
+          if (n < p.N) wgrad_store4(row, n, p.N, block(i, j));
           __builtin_amdgcn_sched_barrier(0);  // block by block: no accumulator hoisted ahead
         }
       }
@@ -452,7 +460,7 @@ __global__ __launch_bounds__(WM * WN * 64, (BM / WM / 16) * (BN / WN / 16) <= 16
       if (m >= p.M || n >= p.N) continue;
       const int64_t off = (int64_t)expert * p.dw_se + m * p.dw_sm;
       if (dw_vec) {
-        *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.dw) + off + n) = t[b];
+        wgrad_store4(reinterpret_cast<float*>(p.dw) + off, n, p.N, t[b]);
       } else if constexpr (!VEC_ONLY) {
         const float e[4] = {t[b].x, t[b].y, t[b].z, t[b].w};
 #pragma unroll
