@@ -88,33 +88,37 @@ static std::atomic<int64_t> g_wgrad_chunk{0};
 void wgrad_geometry(int64_t M, int64_t N, int64_t n_routes, int32_t n_experts, int32_t op_dtype, int64_t* split,
                     int64_t* grid_chunks, int64_t* max_slots, int64_t* tiles_mn) {
   const int64_t bk = op_dtype == kF32 ? 32 : 64;
-  // chunk = max(1024, 6 * mean routes per expert): an expert is split only
-  // when it holds over six times the mean.  Every split adds an fp32 partial
-  // of the expert's dW per chunk, written and read back; measured on the FFN
-  // stack (Zipf-skewed, up to 16x the mean on one expert) the weight gradient
-  // takes 670 / 570 / 516 / 534 / 644 / 710 us per launch at 2 / 4 / 6 / 8 /
-  // 12 / 16 x the mean (unsplit experts beyond that become the last
-  // workgroups to finish); balanced configs do not split at any of them.
+  // chunk = max(1024, one CU's share of the launch: R x tiles / 256 CUs).  A
+  // longer expert alone would outlast the rest of the launch; a shorter chunk
+  // adds an fp32 partial of the expert's dW, written and read back.  Measured
+  // (longest chunk first, cvmm_wgrad_sched.h): ff_up with loads up to 2.2x
+  // the mean, share 2048: 46 us against 51 / 67 / 73 at 1536 / 1280 / 1024
+  // and 57 at 3072; the FFN stack (Zipf loads up to 16x), share 8192: 434 us
+  // per launch against 521 / 462 / 558 at 6144 / 12288 / 16384.
+  int bm, bn;
+  if (op_dtype == kF32) wgrad_tile(M, N, &bm, &bn);
+  else wgrad_fast_tile(M, N, wgrad_auto_tile(M, N, n_experts), &bm, &bn);
+  const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
   const int64_t knob = g_wgrad_chunk.load();
   int64_t s = knob;
   if (s <= 0) {
-    s = n_experts > 0 ? (6 * n_routes + n_experts - 1) / n_experts : n_routes;
+    s = (int64_t)((double)n_routes * (double)tiles / 256.0);
     if (s < 1024) s = 1024;
+    if (s > n_routes && n_routes > 0) s = n_routes;
   }
   s = (s + bk - 1) / bk * bk;
   *split = s;
   *grid_chunks = (n_routes + s - 1) / s + n_experts;
   // a multi-chunk expert has > s routes and < 2*count/s chunks
   *max_slots = (2 * n_routes) / s + 1;
-  int bm, bn;
   wgrad_tile(M, N, &bm, &bn);
   *tiles_mn = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
 }
 
-int32_t wgrad_auto_tile(int64_t M, int64_t N, int64_t grid_chunks) {
+int32_t wgrad_auto_tile(int64_t M, int64_t N, int32_t n_experts) {
   if (M < 256 || N < 256) return kWgTileBase;
   const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
-  return grid_chunks * tiles >= 4 * 256 ? kWgTile256x256W8 : kWgTileBase;
+  return n_experts * tiles >= 2 * 256 ? kWgTile256x256W8 : kWgTileBase;
 }
 
 // fp32 partial elements of one slot: the M x N rounding of the tile the
@@ -1465,23 +1469,26 @@ int cvmm_bwd_w(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld, con
   p.M = d_in; p.N = d_out;
   p.offsets = offs; p.n_experts = n_experts; p.n_routes = n_routes;
   p.dw = grad_keys; p.dw_dtype = grad_keys_dtype; p.dw_se = gk_se; p.dw_sm = gk_si; p.dw_sn = gk_sj;
-  // dW tile: the knob, else 256 x 256 where both sides fill it and the grid
-  // still holds >= 4 workgroups per CU (the FFN stack's 2048 x 512: 1.6 -> 0.8 ms per
-  // launch; the gathered bytes per flop halve against 128 x 128)
+  // dW tile: the knob, else 256 x 256 where both sides fill it and the
+  // experts' tiles fill two rounds of CUs (the FFN stack's 2048 x 512: 1.6 ->
+  // 0.8 ms per launch; 8 experts of 1024 x 4096, two rounds: 161 -> 131 us;
+  // the gathered bytes per flop halve against 128 x 128)
   const int32_t tile = g_wgrad_tile.load();
-  p.tile_choice = tile > 0 ? tile - 1 : wgrad_auto_tile(d_in, d_out, p.grid_chunks);
-  // Workgroup order: the knob, else chunk-xcd for the 16-bit kernel's 128 x
-  // 128 tile (ff_up 38.5 -> 35.0 us, ff_down 52.9 -> 50.8 us per launch: the
-  // eight dW tiles of a chunk share its routes' gradient rows in one L2) and
-  // tile-major for the other tiles (the activation column slice of one tile,
-  // shared by the top-k experts of each token, stays in one XCD's L2:
-  // switch_v 223 us against 249 with chunk-xcd, the FFN stack 4.49 against
-  // 4.55 ms).  Every order gives the same bits.
+  p.tile_choice = tile > 0 ? tile - 1 : wgrad_auto_tile(d_in, d_out, n_experts);
+  // Workgroup order: the knob, else chunk-xcd for square tiles (the dW tiles
+  // of a chunk share its routes' rows in one L2, and the chunks start longest
+  // first, dealt evenly to the XCDs: ff_up with loads up to 2.2x the mean 57
+  // -> 46 us, the FFN stack 481 -> 434, 8 wide experts 131 -> 125) and
+  // tile-major in expert order for the 64-wide tiles (the activation column
+  // slice of one tile, shared by the top-k experts of each token, stays in
+  // one XCD's L2: switch_v 227 us against 274 with chunk-xcd and 255
+  // tile-major by length).  Every order gives the same bits.
   const int32_t order = g_wgrad_order.load();
   if (order == 0) {
     int bm, bn;
     wgrad_fast_tile(d_in, d_out, p.tile_choice, &bm, &bn);
-    p.order = wgrad_fast_eligible(p, op_dtype) && bm == 128 && bn == 128 ? kWgOrderChunkXcd : kWgOrderTile;
+    const bool even = (bm == 128 && bn == 128) || (bm == 256 && bn == 256);
+    p.order = wgrad_fast_eligible(p, op_dtype) && even ? kWgOrderChunkXcd : kWgOrderTile;
   } else {
     p.order = order == 1 ? kWgOrderChunk : order == 3 ? kWgOrderChunkXcd : kWgOrderTile;
   }

@@ -1,0 +1,113 @@
+// Work schedule of the per-expert weight gradients: (expert, route chunk)
+// slots, largest first.
+#pragma once
+
+#include "cvmm_common.h"
+#include "cvmm_internal.h"
+
+namespace cvmm {
+
+struct WgSched {
+  int32_t expert, nch, last;
+  int64_t lo, hi, slot, base_slot;
+};
+
+// Experts the sorted order is computed for (one per thread).
+constexpr int32_t kWgSortExperts = 256;
+
+// (expert, route chunk) of work slot `slot_id`.  An expert of n routes is cut
+// into ceil(n / p.split) chunks of equal length (multiples of 32 routes; at
+// least one chunk per expert).  Slots run over the experts by chunk length,
+// longest first (ties by id), so that the long chunks start first and the
+// short ones fill the end of the launch: a router's loads differ by 2x and
+// more between experts, and in id order the launch ended on whichever expert
+// came last.  More than kWgSortExperts experts keep id order.  Every
+// workgroup computes the same order; `scratch` is 2 * kWgSortExperts ints of
+// LDS, free again when this returns.  Returns false (uniformly) past the last
+// slot.
+template <int NT>
+__device__ __forceinline__ bool wgrad_schedule(const WgradParams& p, int64_t slot_id, WgSched& s, int32_t* scratch, bool by_length) {
+  static_assert(NT >= kWgSortExperts, "one thread per sorted expert");
+  const int tid = threadIdx.x, lane = tid & 63;
+  auto range = [&](int32_t e, int64_t& st, int64_t& n) {
+    st = n = 0;
+    if (e < p.n_experts) {
+      int64_t end = p.offsets[e], start = e > 0 ? p.offsets[e - 1] : 0;
+      end = end < 0 ? 0 : (end > p.n_routes ? p.n_routes : end);
+      start = start < 0 ? 0 : (start > p.n_routes ? p.n_routes : start);
+      st = start;
+      n = end > start ? end - start : 0;
+    }
+  };
+  auto chunks_of = [&](int32_t e, int64_t n) -> int32_t {
+    if (e >= p.n_experts) return 0;
+    const int64_t c = (n + p.split - 1) / p.split;
+    return c < 1 ? 1 : (int32_t)c;
+  };
+  const bool sorted = by_length && p.n_experts <= kWgSortExperts;
+  int32_t* len = scratch;                    // chunk length of expert e
+  int32_t* order = scratch + kWgSortExperts; // expert of rank r
+  if (sorted) {
+    if (tid < kWgSortExperts) {
+      int64_t st, n;
+      range(tid, st, n);
+      const int32_t nch = chunks_of(tid, n);
+      len[tid] = nch > 0 ? (int32_t)((n + nch - 1) / nch) : -1;
+    }
+    __syncthreads();
+    if (tid < p.n_experts) {
+      const int32_t mine = len[tid];
+      int32_t rank = 0;
+      for (int32_t j = 0; j < p.n_experts; j += 4) {  // (entries past the last expert: -1)
+        const int4 o = *reinterpret_cast<const int4*>(len + j);
+        rank += (o.x > mine || (o.x == mine && j < tid)) ? 1 : 0;
+        rank += (o.y > mine || (o.y == mine && j + 1 < tid)) ? 1 : 0;
+        rank += (o.z > mine || (o.z == mine && j + 2 < tid)) ? 1 : 0;
+        rank += (o.w > mine || (o.w == mine && j + 3 < tid)) ? 1 : 0;
+      }
+      order[rank] = tid;
+    }
+    __syncthreads();
+  }
+  if (tid < 64) {
+    if (lane == 0) s.expert = -1;
+    int32_t carry = 0, carry_multi = 0;
+    for (int32_t base = 0; base < p.n_experts; base += 64) {
+      const int32_t r = base + lane;
+      const int32_t e = r < p.n_experts ? (sorted ? order[r] : r) : p.n_experts;
+      int64_t st, n;
+      range(e, st, n);
+      const int32_t nch = chunks_of(e, n);
+      const int32_t multi = nch > 1 ? nch : 0;
+      const int32_t incl = wave_incl_scan(nch) + carry, incl_m = wave_incl_scan(multi) + carry_multi;
+      const int32_t excl = incl - nch;
+      if (nch > 0 && slot_id >= excl && slot_id < incl) {
+        const int64_t c = slot_id - excl;
+        const int64_t step = ((n + nch - 1) / nch + 31) / 32 * 32;
+        const int64_t a = c * step < n ? c * step : n, b = (c + 1) * step < n && c + 1 < nch ? (c + 1) * step : n;
+        s.expert = e;
+        s.nch = nch;
+        s.lo = st + a;
+        s.hi = st + b;
+        s.base_slot = incl_m - multi;
+        s.slot = s.base_slot + c;
+      }
+      carry = __builtin_amdgcn_readlane(incl, 63);
+      carry_multi = __builtin_amdgcn_readlane(incl_m, 63);
+      if (slot_id < carry) break;
+    }
+  }
+  __syncthreads();
+  return s.expert >= 0;
+}
+
+// Chunk-per-XCD order: (slot, tile) of workgroup i where the tiles of one
+// chunk run together on one XCD (i % 8) and ranks are dealt to the XCDs back
+// and forth (0 .. 7, 7 .. 0), which evens their sums.
+__device__ __forceinline__ void wgrad_chunk_xcd(uint32_t i, uint32_t tiles, int64_t* slot_id, int64_t* tile) {
+  const uint32_t xcd = i % 8, local = i / 8, row = local / tiles;
+  *slot_id = (int64_t)row * 8 + ((row & 1) ? 7 - xcd : xcd);
+  *tile = local - row * tiles;
+}
+
+}  // namespace cvmm

@@ -32,8 +32,11 @@
 //    of 128 x 64 (two waves per SIMD: the FFN stack's launch 514 -> 485 us).
 //    Every tile sums each dW element over the same slices in the same
 //    order, so the tile choice never changes bits.
-// Workgroup orders (WgradParams::order): tile-major by default; chunk-major
-// and chunk-per-XCD for tuning.
+// Workgroup orders (WgradParams::order): chunk-per-XCD, longest chunks first,
+// for square tiles; tile-major for the 64-wide ones; chunk-major for tuning.
+// (Two groups of four waves alternating reads and MFMAs between barriers, as
+// against all eight in step: 434 -> 468 us per launch at the FFN stack; with
+// the MFMAs left out the loop takes 363, with the DMA left out 370.)
 // LDS rows are swizzled at 16-byte granularity so that a transposed read's
 // 16 lanes (4 routes x 32 bytes) hit distinct banks:
 //   256-byte rows: chunk ^ (2 * ((row & 3) | (((row >> 3) & 1) << 2)))
@@ -42,6 +45,7 @@
 #pragma once
 
 #include "cvmm_gemm_panel.h"
+#include "cvmm_wgrad_sched.h"
 
 namespace cvmm {
 
@@ -84,52 +88,6 @@ struct Wg3Cfg {
   static_assert(TBL >= 256, "route table");
 };
 
-struct Wg3Sched {
-  int32_t expert, nch, last;
-  int64_t lo, hi, slot, base_slot;
-};
-
-// (expert, route chunk) of work slot `slot_id`: experts in order, each cut
-// into chunks of p.split routes (at least one chunk per expert).
-__device__ __forceinline__ bool wgrad_schedule(const WgradParams& p, int64_t slot_id, Wg3Sched& s) {
-  const int lane = threadIdx.x & 63;
-  if (threadIdx.x < 64) {
-    if (lane == 0) s.expert = -1;
-    int64_t carry = 0, carry_multi = 0;
-    for (int32_t base = 0; base < p.n_experts; base += 64) {
-      const int32_t e = base + lane;
-      int64_t start = 0, end = 0, nch = 0;
-      if (e < p.n_experts) {
-        end = p.offsets[e];
-        start = e > 0 ? p.offsets[e - 1] : 0;
-        end = end < 0 ? 0 : (end > p.n_routes ? p.n_routes : end);
-        start = start < 0 ? 0 : (start > p.n_routes ? p.n_routes : start);
-        if (end < start) end = start;
-        nch = (end - start + p.split - 1) / p.split;
-        if (nch < 1) nch = 1;
-      }
-      const int64_t multi = nch > 1 ? nch : 0;
-      const int64_t incl = wave_incl_scan(nch) + carry;
-      const int64_t incl_m = wave_incl_scan(multi) + carry_multi;
-      const int64_t excl = incl - nch;
-      if (e < p.n_experts && slot_id >= excl && slot_id < incl) {
-        const int64_t c = slot_id - excl;
-        s.expert = e;
-        s.nch = (int32_t)nch;
-        s.lo = start + c * p.split;
-        s.hi = (start + (c + 1) * p.split) < end ? start + (c + 1) * p.split : end;
-        s.base_slot = incl_m - multi;
-        s.slot = s.base_slot + c;
-      }
-      carry = __shfl(incl, 63, 64);
-      carry_multi = __shfl(incl_m, 63, 64);
-      if (slot_id < carry) break;
-    }
-  }
-  __syncthreads();
-  return s.expert >= 0;
-}
-
 // dW of fp32 rows: a lane's 4 columns are one store (at any alignment; the
 // row's last piece may be shorter).
 __host__ __device__ inline bool wgrad_dw_vec(const WgradParams& p) { return p.dw_sn == 1 && p.dw_dtype == kF32; }
@@ -157,7 +115,7 @@ __global__ __launch_bounds__(WM * WN * 64, (BM / WM / 16) * (BN / WN / 16) <= 16
   __shared__ __attribute__((aligned(16))) int32_t t_x[TBL];
   __shared__ __attribute__((aligned(16))) int32_t t_g[TBL];
   __shared__ __attribute__((aligned(16))) float t_w[WEIGHTED ? TBL : 4];
-  __shared__ Wg3Sched sched;
+  __shared__ WgSched sched;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -166,9 +124,7 @@ __global__ __launch_bounds__(WM * WN * 64, (BM / WM / 16) * (BN / WN / 16) <= 16
   const int64_t tiles = ((p.M + BM - 1) / BM) * tiles_n;
   int64_t slot_id, tile;
   if (p.order == kWgOrderChunkXcd) {  // grid = round_up(grid_chunks, 8) * tiles
-    const int64_t xcd = blockIdx.x % 8, local = blockIdx.x / 8;
-    slot_id = (local / tiles) * 8 + xcd;
-    tile = local % tiles;
+    wgrad_chunk_xcd(blockIdx.x, (uint32_t)tiles, &slot_id, &tile);
   } else {
     const int64_t id = xcd_remap(blockIdx.x, gridDim.x);
     slot_id = p.order == kWgOrderTile ? id % p.grid_chunks : id / tiles;
@@ -176,10 +132,12 @@ __global__ __launch_bounds__(WM * WN * 64, (BM / WM / 16) * (BN / WN / 16) <= 16
   }
   const int64_t m0 = (tile / tiles_n) * BM, n0 = (tile % tiles_n) * BN;
 
-  if (!wgrad_schedule(p, slot_id, sched)) return;
-  const int32_t expert = sched.expert;
+  if (!wgrad_schedule<Cfg::NT>(p, slot_id, sched, reinterpret_cast<int32_t*>(ring),
+                               p.order == kWgOrderChunkXcd))
+    return;
+  const int32_t expert = __builtin_amdgcn_readfirstlane(sched.expert);
   const int64_t lo = sched.lo, hi = sched.hi;
-  const int32_t nch = sched.nch;
+  const int32_t nch = __builtin_amdgcn_readfirstlane(sched.nch);
 
   // ---- DMA geometry: instruction j of this wave fills slice bytes
   // [(wave * D + j) * 1024, +1024): x rows (TA) first, then dY rows (TB)

@@ -96,12 +96,13 @@ int cvmm_timing_result(uint32_t kernel_class, double* total_ms, int64_t* launche
  *   CVMM_TUNE_WGRAD_ORDER: workgroup order of the weight-gradient kernel,
  *     1 = the tiles of one expert chunk on one XCD, 2 = one dW tile of every
  *     expert on one XCD, 3 = expert chunk c on XCD c % 8 with all its tiles.
- *     Built in: 3 for the 16-bit kernel's 128 x 128 dW tile, else 2.
+ *     Built in: 3 for the 16-bit kernel's 128 x 128 and 256 x 256 dW tiles
+ *     (3 starts the longest chunks first, in up to 256 experts), else 2.
  *   CVMM_TUNE_WGRAD_TILE: dW tile of the 16-bit weight-gradient kernel where
  *     its base tile is 128 x 128 and dW is contiguous aligned fp32: 1 = 128 x
  *     128, 2 = 256 x 128, 3 = 128 x 256, 4 = 256 x 256 of four waves, 5 =
  *     256 x 256 of eight waves.  Built in: 256 x 256 of eight waves when
- *     d_in, d_out >= 256 and the grid holds >= 4 tiles per CU.
+ *     d_in, d_out >= 256 and the experts' tiles fill two rounds of 256 CUs.
  *   CVMM_TUNE_GEMM_ORDER: m-tile order of the routed GEMMs (forward, grad
  *     input), 1 = expert-major, 2 = token-major (tile j of every expert next
  *     to each other; up to 256 experts).  Built in: token-major for the
@@ -120,8 +121,8 @@ int cvmm_timing_result(uint32_t kernel_class, double* total_ms, int64_t* launche
  *   CVMM_TUNE_WGRAD_CHUNK: routes per chunk of the weight gradient's split
  *     reduction (rounded up to the kernel's 32- or 64-route slices; an
  *     expert with more routes is split into chunks whose fp32 partials are
- *     summed in chunk order).  Built in: max(1024, 6 x the mean routes per
- *     expert).  Workspace queries depend on it: query after setting it.
+ *     summed in chunk order).  Built in: max(1024, one CU's share of the
+ *     launch, routes x dW tiles / 256).  Workspace queries depend on it: query after setting it.
  *   CVMM_TUNE_RING_TILE: tile of the long-K routed GEMM (K > 128, N > 64):
  *     1 = 128 x 128, 2 = 160 x 128, 3 = 256 x 256 of eight waves where N is
  *     a multiple of 256 (elsewhere the built-in height).  Built in: 256 x
