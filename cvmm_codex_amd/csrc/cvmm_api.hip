@@ -48,6 +48,7 @@ static bool routed_gemm_is_panel(const GemmParams& p, int32_t op) {
 }
 
 hipError_t launch_routed_gemm(const GemmParams& p, int32_t op, hipStream_t s) {
+  if (f32_gemm_eligible(p, op)) return launch_f32_gemm(p, s);
   if (small_gemm_eligible(p, op)) return launch_routed_small(p, s);
   if (routed_gemm_decode_applies(p, op)) return launch_routed_gemm_decode(p, op, s);
   if (nt_eligible(p, op)) return op == kBF16 ? launch_routed_gemm_nt_bf16(p, s) : launch_routed_gemm_nt_f16(p, s);
@@ -70,6 +71,7 @@ static bool wgrad_fast_eligible(const WgradParams& p, int32_t op) {
 }
 
 hipError_t launch_wgrad(const WgradParams& p, int32_t op, hipStream_t s) {
+  if (f32_wgrad_eligible(p, op)) return launch_f32_wgrad(p, s);
   if (small_wgrad_eligible(p, op)) return launch_wgrad_small(p, s);
   if (wgrad_fast_eligible(p, op)) return op == kBF16 ? launch_wgrad_v3_bf16(p, s) : launch_wgrad_v3_f16(p, s);
   if (op == kBF16) return launch_wgrad_bf16(p, s);
@@ -96,7 +98,7 @@ void wgrad_geometry(int64_t M, int64_t N, int64_t n_routes, int32_t n_experts, i
   // and 57 at 3072; the FFN stack (Zipf loads up to 16x), share 8192: 434 us
   // per launch against 521 / 462 / 558 at 6144 / 12288 / 16384.
   int bm, bn;
-  if (op_dtype == kF32) wgrad_tile(M, N, &bm, &bn);
+  if (op_dtype == kF32) f32_wgrad_tile(M, N, n_experts, &bm, &bn);
   else wgrad_fast_tile(M, N, wgrad_auto_tile(M, N, n_experts), &bm, &bn);
   const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
   const int64_t knob = g_wgrad_chunk.load();
@@ -112,6 +114,7 @@ void wgrad_geometry(int64_t M, int64_t N, int64_t n_routes, int32_t n_experts, i
   // a multi-chunk expert has > s routes and < 2*count/s chunks
   *max_slots = (2 * n_routes) / s + 1;
   wgrad_tile(M, N, &bm, &bn);
+  if (op_dtype == kF32) bm = bn = 64;  // the finest fp32 tile (cvmm_f32.hip)
   *tiles_mn = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
 }
 

@@ -147,6 +147,12 @@ hipError_t launch_routed_small(const GemmParams& p, hipStream_t stream);
 bool small_wgrad_eligible(const WgradParams& p, int32_t op);
 hipError_t launch_wgrad_small(const WgradParams& p, hipStream_t stream);
 
+// fp32 products with DMA-staged rows on the matrix cores (cvmm_f32.hip).
+bool f32_gemm_eligible(const GemmParams& p, int32_t op);
+hipError_t launch_f32_gemm(const GemmParams& p, hipStream_t stream);
+bool f32_wgrad_eligible(const WgradParams& p, int32_t op);
+hipError_t launch_f32_wgrad(const WgradParams& p, hipStream_t stream);
+
 // Weight-gradient workgroup orders.  The hardware places workgroup i on XCD
 // i % 8; each XCD has its own L2.
 //   chunk-major:  the tiles of one route chunk adjacent, contiguous ranges of
@@ -188,6 +194,8 @@ int64_t wgrad_partial_elems(int64_t M, int64_t N);
 // built-in tile choice (no knob): 256 x 256 of eight waves where M, N >= 256
 // and the experts' tiles fill two rounds of 256 CUs, else the base tile
 int32_t wgrad_auto_tile(int64_t M, int64_t N, int32_t n_experts);
+// the fp32 kernel's dW tile (cvmm_f32.hip)
+void f32_wgrad_tile(int64_t M, int64_t N, int32_t n_experts, int* bm, int* bn);
 
 // ---------------------------------------------------------------------------
 // selector preparation
