@@ -201,3 +201,30 @@ def test_gate_logits_against_the_torch_projection(T, D, E, amp):
     xo = xd.double().cpu()
     dlo = dl.to(y0.dtype).double().cpu()
     assert norm_rel(to_np(dg1), (xo.t() @ dlo).numpy()) <= tol
+
+
+@pytest.mark.parametrize("T,E,k", [(1, 1, 1), (1, 64, 8), (4, 128, 8), (64, 128, 8), (8, 1024, 64), (9, 100, 64),
+                                   (512, 3, 1), (513, 3, 1), (170, 33, 3), (171, 33, 3), (65, 128, 8)])
+def test_router_sort_around_one_workgroup(T, E, k):
+    """The router that sorts its own routes (up to one chunk of 512 routes in
+    whole tokens) and the two-launch form past it: the selector equals the
+    stable sort of the returned ids."""
+    g = torch.Generator().manual_seed(T + E + k)
+    logits = torch.randn(T, E, generator=g)
+    logits[T // 2] = 1.0   # ties: lower ids first
+    w, sel, s = C.cvmm_route_topk(logits.cuda(), k, True)
+    flat = sel.reshape(-1).cpu()
+    ssel, perm = torch.sort(flat, stable=True)
+    s._resolve(E)
+    assert torch.equal(s.sel.reshape(-1).cpu().long(), ssel)
+    assert torch.equal(s.out_index.cpu(), perm)
+    assert torch.equal(s.sel_index.cpu(), perm // k)
+    pos = torch.empty_like(perm)
+    pos[perm] = torch.arange(T * k)
+    assert torch.equal(s.out_index._cvmm_route_pos.cpu().long(), pos)
+    offsets = s._routing.by_e[E][3]
+    assert torch.equal(offsets.cpu(), torch.bincount(flat, minlength=E).cumsum(0))
+    p = torch.softmax(logits, -1).gather(1, sel.cpu())
+    ref = p / p.sum(-1, keepdim=True).clamp_min(1e-20)
+    assert torch.allclose(w.cpu(), ref, rtol=1e-5, atol=1e-7)
+    assert torch.equal(sel[T // 2].cpu(), torch.arange(k))
