@@ -34,6 +34,7 @@ from dataclasses import dataclass
 from typing import Dict, NamedTuple, Optional, Tuple, Union
 
 import torch
+from torch.autograd import forward_ad as _forward_ad
 
 from . import _native as N
 from . import compile_ops as _ops
@@ -538,6 +539,36 @@ def cvmm_prepare_sel2(sel: Union[torch.Tensor, CVMMSel], w: Optional[torch.Tenso
 
 
 # ----------------------------------------------------------------------------
+# autograd functions of inference calls
+# ----------------------------------------------------------------------------
+
+class _NoGraph:
+    """The context of an autograd Function's forward that is called by itself:
+    nothing is saved and no gradient is needed."""
+
+    needs_input_grad = (False,) * 8
+
+    def save_for_backward(self, *tensors):
+        pass
+
+    mark_non_differentiable = save_for_backward
+
+    def set_materialize_grads(self, value):
+        pass
+
+
+def _apply(fn, *args):
+    """fn.apply(*args); without a graph to record -- grad mode off, no
+    forward-mode level and no function transform active -- fn's forward by
+    itself (three of these calls per inference block cost ~5 us of host time
+    each, of the ~120 us a four-token decode step takes the host)."""
+    if (torch.is_grad_enabled() or _forward_ad._current_level >= 0
+            or torch._C._are_functorch_transforms_active()):
+        return fn.apply(*args)
+    return fn.forward(_NoGraph(), *args)
+
+
+# ----------------------------------------------------------------------------
 # router
 # ----------------------------------------------------------------------------
 
@@ -592,7 +623,7 @@ def cvmm_route_topk(logits: torch.Tensor, k: int, renormalize: bool = True):
     if _compiling():
         w, sel, ssel, perm, tok, offsets, route_pos = _ops.route_topk(logits, k, renormalize)
     else:
-        w, sel, ssel, perm, tok, offsets, route_pos = _RouteTopK.apply(logits, k, renormalize)
+        w, sel, ssel, perm, tok, offsets, route_pos = _apply(_RouteTopK, logits, k, renormalize)
         perm._cvmm_route_pos = route_pos
     sel = sel.view(*lead, k)
     routing = _Routing(sel.reshape(-1), k)
@@ -665,11 +696,10 @@ def cvmm_gate_logits(x: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     if gate.dim() != 2 or x.shape[-1] != gate.shape[0]:
         raise ValueError(f"cvmm_gate_logits: x {tuple(x.shape)} and gate {tuple(gate.shape)} do not multiply")
     if torch.is_autocast_enabled("cuda"):
-        op = torch.get_autocast_dtype("cuda")
-    else:
-        op = torch.result_type(x, gate)
-    with torch.autocast("cuda", enabled=False):
-        return _GateLogits.apply(x, gate, op)
+        # both operands reach the product in the autocast dtype, which
+        # autocast leaves as they are
+        return _apply(_GateLogits, x, gate, torch.get_autocast_dtype("cuda"))
+    return _apply(_GateLogits, x, gate, torch.result_type(x, gate))
 
 
 # ----------------------------------------------------------------------------
@@ -865,7 +895,7 @@ def cvmm_gelu(x: torch.Tensor, sel: Union[torch.Tensor, CVMMSel], keys: torch.Te
                             not sel._route_mode, torch.is_grad_enabled() and x.requires_grad)
         cast = (keys, op, plan) if plan.casts else None
     sel._resolve(keys.shape[0], cast)
-    return CVMMGelu.apply(x, sel._raw_shape_tensor(), sel.sel_index, sel.sel, keys, sel.out_index)
+    return _apply(CVMMGelu, x, sel._raw_shape_tensor(), sel.sel_index, sel.sel, keys, sel.out_index)
 
 
 known_shapes = set()

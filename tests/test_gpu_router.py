@@ -228,3 +228,32 @@ def test_router_sort_around_one_workgroup(T, E, k):
     ref = p / p.sum(-1, keepdim=True).clamp_min(1e-20)
     assert torch.allclose(w.cpu(), ref, rtol=1e-5, atol=1e-7)
     assert torch.equal(sel[T // 2].cpu(), torch.arange(k))
+
+
+def test_inference_calls_match_recorded_ones():
+    """Without a graph to record, the router, gate and GELU calls run their
+    forwards by themselves: the results of the recorded calls, bit for bit,
+    in no_grad and inference mode; a forward-mode level still refuses."""
+    g = torch.Generator().manual_seed(0)
+    T, D, H, E, k = 37, 256, 64, 16, 4
+    x = torch.randn(T, D, generator=g).to(torch.bfloat16).cuda()
+    gate = (torch.randn(D, E, generator=g) / 16).cuda()
+    keys = (torch.randn(E, D, H, generator=g) / 16).cuda()
+
+    def block():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            logits = C.cvmm_gate_logits(x, gate)
+            w, sel, s = C.cvmm_route_topk(logits, k, True)
+            return logits, w, sel, C.cvmm_gelu(x, s, keys)
+
+    rec = block()
+    for mode in (torch.no_grad, torch.inference_mode):
+        with mode():
+            got = block()
+        assert not any(t.requires_grad for t in got)
+        for a, b in zip(got, rec):
+            assert torch.equal(a, b)
+    with torch.no_grad(), torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x.float(), torch.ones_like(x, dtype=torch.float32))
+        with pytest.raises(Exception):
+            C.cvmm_gate_logits(dual, gate)
