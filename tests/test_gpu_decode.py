@@ -37,7 +37,7 @@ def _check(y, ref, tol=2e-2):
 @pytest.mark.parametrize("T,k,E,D,H,hot", [
     (1, 1, 1, 8, 8, False), (1, 8, 64, 1024, 128, False), (4, 8, 64, 128, 1024, False), (3, 2, 5, 40, 72, False),
     (17, 1, 1, 136, 136, False), (33, 8, 16, 200, 520, True), (65, 4, 8, 1000, 264, True), (64, 2, 3, 264, 64, False),
-    (200, 4, 16, 96, 136, True), (130, 8, 128, 520, 40, True)])
+    (200, 4, 16, 96, 136, True), (130, 8, 128, 520, 40, True), (20, 4, 70, 1000, 1032, True)])
 def test_forward_reads_the_stored_weights(T, k, E, D, H, hot, op, weights):
     x, keys, sel = _case(T, k, E, D, H, op, weights, hot, T + D)
     with torch.no_grad(), torch.autocast("cuda", dtype=_DT[op]):
