@@ -12,8 +12,10 @@ struct WgSched {
   int64_t lo, hi, slot, base_slot;
 };
 
-// Experts the sorted order is computed for (one per thread).
+// Experts the sorted order is computed for (one per thread), and the mean
+// routes per expert from which it is.
 constexpr int32_t kWgSortExperts = 256;
+constexpr int64_t kWgSortRoutes = 128;
 
 // (expert, route chunk) of work slot `slot_id`.  An expert of n routes is cut
 // into ceil(n / p.split) chunks of equal length (multiples of 32 routes; at
@@ -21,8 +23,10 @@ constexpr int32_t kWgSortExperts = 256;
 // longest first (ties by id), so that the long chunks start first and the
 // short ones fill the end of the launch: a router's loads differ by 2x and
 // more between experts, and in id order the launch ended on whichever expert
-// came last.  More than kWgSortExperts experts keep id order.  Every
-// workgroup computes the same order; `scratch` is 2 * kWgSortExperts ints of
+// came last.  More than kWgSortExperts experts keep id order, and so do
+// launches of few routes per expert, where the order costs every workgroup
+// more than it evens out (18 routes on each of 122 experts: 38 us against 29
+// per launch).  Every workgroup computes the same order; `scratch` is 2 * kWgSortExperts ints of
 // LDS, free again when this returns.  Returns false (uniformly) past the last
 // slot.
 template <int NT>
@@ -44,7 +48,7 @@ __device__ __forceinline__ bool wgrad_schedule(const WgradParams& p, int64_t slo
     const int64_t c = (n + p.split - 1) / p.split;
     return c < 1 ? 1 : (int32_t)c;
   };
-  const bool sorted = by_length && p.n_experts <= kWgSortExperts;
+  const bool sorted = by_length && p.n_experts <= kWgSortExperts && p.n_routes >= kWgSortRoutes * p.n_experts;
   int32_t* len = scratch;                    // chunk length of expert e
   int32_t* order = scratch + kWgSortExperts; // expert of rank r
   if (sorted) {
@@ -58,12 +62,18 @@ __device__ __forceinline__ bool wgrad_schedule(const WgradParams& p, int64_t slo
     if (tid < p.n_experts) {
       const int32_t mine = len[tid];
       int32_t rank = 0;
-      for (int32_t j = 0; j < p.n_experts; j += 4) {  // (entries past the last expert: -1)
-        const int4 o = *reinterpret_cast<const int4*>(len + j);
-        rank += (o.x > mine || (o.x == mine && j < tid)) ? 1 : 0;
-        rank += (o.y > mine || (o.y == mine && j + 1 < tid)) ? 1 : 0;
-        rank += (o.z > mine || (o.z == mine && j + 2 < tid)) ? 1 : 0;
-        rank += (o.w > mine || (o.w == mine && j + 3 < tid)) ? 1 : 0;
+      for (int32_t j = 0; j < p.n_experts; j += 16) {  // (entries past the last expert: -1)
+        int4 o[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) o[q] = *reinterpret_cast<const int4*>(len + j + 4 * q);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int32_t at = j + 4 * q;
+          rank += (o[q].x > mine || (o[q].x == mine && at < tid)) ? 1 : 0;
+          rank += (o[q].y > mine || (o[q].y == mine && at + 1 < tid)) ? 1 : 0;
+          rank += (o[q].z > mine || (o[q].z == mine && at + 2 < tid)) ? 1 : 0;
+          rank += (o[q].w > mine || (o[q].w == mine && at + 3 < tid)) ? 1 : 0;
+        }
       }
       order[rank] = tid;
     }
