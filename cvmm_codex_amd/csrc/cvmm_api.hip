@@ -99,7 +99,7 @@ void wgrad_geometry(int64_t M, int64_t N, int64_t n_routes, int32_t n_experts, i
   // per launch against 521 / 462 / 558 at 6144 / 12288 / 16384.
   int bm, bn;
   if (op_dtype == kF32) f32_wgrad_tile(M, N, n_experts, &bm, &bn);
-  else wgrad_fast_tile(M, N, wgrad_auto_tile(M, N, n_experts), &bm, &bn);
+  else wgrad_fast_tile(M, N, wgrad_auto_tile(M, N, n_routes, n_experts), &bm, &bn);
   const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
   const int64_t knob = g_wgrad_chunk.load();
   int64_t s = knob;
@@ -118,10 +118,18 @@ void wgrad_geometry(int64_t M, int64_t N, int64_t n_routes, int32_t n_experts, i
   *tiles_mn = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
 }
 
-int32_t wgrad_auto_tile(int64_t M, int64_t N, int32_t n_experts) {
+int32_t wgrad_auto_tile(int64_t M, int64_t N, int64_t n_routes, int32_t n_experts) {
   if (M < 256 || N < 256) return kWgTileBase;
-  const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
-  return n_experts * tiles >= 2 * 256 ? kWgTile256x256W8 : kWgTileBase;
+  const int64_t m = (M + 255) / 256, n = (N + 255) / 256;
+  const int64_t wide = n_experts * m * n;
+  if (7 * wide >= 6 * 4 * 256) return kWgTile256x256W8;
+  // two rounds of CUs where the experts are long and the wide tiles cover
+  // little more than the base ones (8 experts of 1024 x 4096, 1024 routes
+  // each: 161 -> 131 us; 37 routes on each of 47 experts of 1344 x 288: 40
+  // us against 28)
+  const int64_t base = ((M + 127) / 128) * ((N + 127) / 128);
+  return wide >= 2 * 256 && n_routes >= 512 * (int64_t)n_experts && 20 * 4 * m * n <= 23 * base ? kWgTile256x256W8
+                                                                                                 : kWgTileBase;
 }
 
 // fp32 partial elements of one slot: the M x N rounding of the tile the
@@ -1477,7 +1485,7 @@ int cvmm_bwd_w(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld, con
   // 0.8 ms per launch; 8 experts of 1024 x 4096, two rounds: 161 -> 131 us;
   // the gathered bytes per flop halve against 128 x 128)
   const int32_t tile = g_wgrad_tile.load();
-  p.tile_choice = tile > 0 ? tile - 1 : wgrad_auto_tile(d_in, d_out, n_experts);
+  p.tile_choice = tile > 0 ? tile - 1 : wgrad_auto_tile(d_in, d_out, n_routes, n_experts);
   // Workgroup order: the knob, else chunk-xcd for square tiles (the dW tiles
   // of a chunk share its routes' rows in one L2, and the chunks start longest
   // first, dealt evenly to the XCDs: ff_up with loads up to 2.2x the mean 57

@@ -192,8 +192,9 @@ void wgrad_geometry(int64_t M, int64_t N, int64_t n_routes, int32_t n_experts, i
                     int64_t* split, int64_t* grid_chunks, int64_t* max_slots, int64_t* tiles_mn);
 int64_t wgrad_partial_elems(int64_t M, int64_t N);
 // built-in tile choice (no knob): 256 x 256 of eight waves where M, N >= 256
-// and the experts' tiles fill two rounds of 256 CUs, else the base tile
-int32_t wgrad_auto_tile(int64_t M, int64_t N, int32_t n_experts);
+// and the experts' tiles fill about four rounds of 256 CUs, or two with long
+// experts, else the base tile
+int32_t wgrad_auto_tile(int64_t M, int64_t N, int64_t n_routes, int32_t n_experts);
 // the fp32 kernel's dW tile (cvmm_f32.hip)
 void f32_wgrad_tile(int64_t M, int64_t N, int32_t n_experts, int* bm, int* bn);
 

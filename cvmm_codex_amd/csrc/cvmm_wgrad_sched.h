@@ -15,7 +15,7 @@ struct WgSched {
 // Experts the sorted order is computed for (one per thread), and the mean
 // routes per expert from which it is.
 constexpr int32_t kWgSortExperts = 256;
-constexpr int64_t kWgSortRoutes = 128;
+constexpr int64_t kWgSortRoutes = 384;
 
 // (expert, route chunk) of work slot `slot_id`.  An expert of n routes is cut
 // into ceil(n / p.split) chunks of equal length (multiples of 32 routes; at
@@ -26,7 +26,7 @@ constexpr int64_t kWgSortRoutes = 128;
 // came last.  More than kWgSortExperts experts keep id order, and so do
 // launches of few routes per expert, where the order costs every workgroup
 // more than it evens out (18 routes on each of 122 experts: 38 us against 29
-// per launch).  Every workgroup computes the same order; `scratch` is 2 * kWgSortExperts ints of
+// per launch; 330 on each of 40, evenly loaded: 16.1 against 14.7).  Every workgroup computes the same order; `scratch` is 2 * kWgSortExperts ints of
 // LDS, free again when this returns.  Returns false (uniformly) past the last
 // slot.
 template <int NT>

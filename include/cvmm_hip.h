@@ -102,7 +102,8 @@ int cvmm_timing_result(uint32_t kernel_class, double* total_ms, int64_t* launche
  *     its base tile is 128 x 128 and dW is contiguous aligned fp32: 1 = 128 x
  *     128, 2 = 256 x 128, 3 = 128 x 256, 4 = 256 x 256 of four waves, 5 =
  *     256 x 256 of eight waves.  Built in: 256 x 256 of eight waves when
- *     d_in, d_out >= 256 and the experts' tiles fill two rounds of 256 CUs.
+ *     d_in, d_out >= 256 and the experts' tiles fill about four rounds of
+ *     256 CUs, or two with >= 512 routes per expert.
  *   CVMM_TUNE_GEMM_ORDER: m-tile order of the routed GEMMs (forward, grad
  *     input), 1 = expert-major, 2 = token-major (tile j of every expert next
  *     to each other; up to 256 experts).  Built in: token-major for the
