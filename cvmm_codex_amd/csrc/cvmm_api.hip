@@ -1481,8 +1481,8 @@ int cvmm_bwd_w(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld, con
   p.offsets = offs; p.n_experts = n_experts; p.n_routes = n_routes;
   p.dw = grad_keys; p.dw_dtype = grad_keys_dtype; p.dw_se = gk_se; p.dw_sm = gk_si; p.dw_sn = gk_sj;
   // dW tile: the knob, else 256 x 256 where both sides fill it and the
-  // experts' tiles fill two rounds of CUs (the FFN stack's 2048 x 512: 1.6 ->
-  // 0.8 ms per launch; 8 experts of 1024 x 4096, two rounds: 161 -> 131 us;
+  // experts' tiles fill the CUs (wgrad_auto_tile; the FFN stack's 2048 x 512:
+  // 1.6 -> 0.8 ms per launch; 8 experts of 1024 x 4096, two rounds: 161 -> 131 us;
   // the gathered bytes per flop halve against 128 x 128)
   const int32_t tile = g_wgrad_tile.load();
   p.tile_choice = tile > 0 ? tile - 1 : wgrad_auto_tile(d_in, d_out, n_routes, n_experts);

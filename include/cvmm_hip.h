@@ -123,12 +123,14 @@ int cvmm_timing_result(uint32_t kernel_class, double* total_ms, int64_t* launche
  *     reduction (rounded up to the kernel's 32- or 64-route slices; an
  *     expert with more routes is split into chunks whose fp32 partials are
  *     summed in chunk order).  Built in: max(1024, one CU's share of the
- *     launch, routes x dW tiles / 256).  Workspace queries depend on it: query after setting it.
+ *     launch, routes x dW tiles / 256).  Workspace queries depend on it:
+ *     query after setting it.
  *   CVMM_TUNE_RING_TILE: tile of the long-K routed GEMM (K > 128, N > 64):
  *     1 = 128 x 128, 2 = 160 x 128, 3 = 256 x 256 of eight waves where N is
  *     a multiple of 256 (elsewhere the built-in height).  Built in: 256 x
- *     256 where it applies and the grid fills two rounds of 256 CUs (the
- *     FFN stack); else 160 rows
+ *     256 where it applies, the grid fills two rounds of 256 CUs and the
+ *     256-row tiles would cover at most 1.2 times the rows of 128-row ones
+ *     (the FFN stack); else 160 rows
  *     unless the estimated dispatch rounds times the tile height come out
  *     more than 5 % higher (the ff_up forward: one round of ~442 tiles
  *     instead of 544 tiles on 512 slots).  All give the same bits. */
