@@ -26,11 +26,14 @@ constexpr int64_t kWgSortRoutes = 384;
 // came last.  More than kWgSortExperts experts keep id order, and so do
 // launches of few routes per expert, where the order costs every workgroup
 // more than it evens out (18 routes on each of 122 experts: 38 us against 29
-// per launch; 330 on each of 40, evenly loaded: 16.1 against 14.7).  Every workgroup computes the same order; `scratch` is 2 * kWgSortExperts ints of
-// LDS, free again when this returns.  Returns false (uniformly) past the last
+// per launch; 330 on each of 40, evenly loaded: 16.1 against 14.7) and those where no expert has more than
+// 1.25 times the mean (1024 routes on each of 64, 1024 x 128: 38.2 us sorted,
+// 36.0 by this test, 34.8 with no test).  Every workgroup computes the same
+// order; `scratch` is 2 * kWgSortExperts ints of LDS, free again when this returns.  Returns false (uniformly) past the last
 // slot.
 template <int NT>
-__device__ __forceinline__ bool wgrad_schedule(const WgradParams& p, int64_t slot_id, WgSched& s, int32_t* scratch, bool by_length) {
+__device__ __forceinline__ bool wgrad_schedule(const WgradParams& p, int64_t slot_id, WgSched& s, int32_t* scratch,
+                                               bool by_length) {
   static_assert(NT >= kWgSortExperts, "one thread per sorted expert");
   const int tid = threadIdx.x, lane = tid & 63;
   auto range = [&](int32_t e, int64_t& st, int64_t& n) {
@@ -48,18 +51,20 @@ __device__ __forceinline__ bool wgrad_schedule(const WgradParams& p, int64_t slo
     const int64_t c = (n + p.split - 1) / p.split;
     return c < 1 ? 1 : (int32_t)c;
   };
-  const bool sorted = by_length && p.n_experts <= kWgSortExperts && p.n_routes >= kWgSortRoutes * p.n_experts;
+  bool sorted = by_length && p.n_experts <= kWgSortExperts && p.n_routes >= kWgSortRoutes * p.n_experts;
   int32_t* len = scratch;                    // chunk length of expert e
   int32_t* order = scratch + kWgSortExperts; // expert of rank r
   if (sorted) {
+    int32_t uneven = 0;
     if (tid < kWgSortExperts) {
       int64_t st, n;
       range(tid, st, n);
       const int32_t nch = chunks_of(tid, n);
       len[tid] = nch > 0 ? (int32_t)((n + nch - 1) / nch) : -1;
+      uneven = 4 * n * p.n_experts > 5 * p.n_routes;
     }
-    __syncthreads();
-    if (tid < p.n_experts) {
+    sorted = __syncthreads_or(uneven) != 0;  // (a barrier: len is written)
+    if (sorted && tid < p.n_experts) {
       const int32_t mine = len[tid];
       int32_t rank = 0;
       for (int32_t j = 0; j < p.n_experts; j += 16) {  // (entries past the last expert: -1)
@@ -77,7 +82,7 @@ __device__ __forceinline__ bool wgrad_schedule(const WgradParams& p, int64_t slo
       }
       order[rank] = tid;
     }
-    __syncthreads();
+    if (sorted) __syncthreads();
   }
   if (tid < 64) {
     if (lane == 0) s.expert = -1;
