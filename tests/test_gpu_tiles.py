@@ -41,3 +41,23 @@ def test_surplus_tiles_zero_the_unrouted_rows(E):
     ref = torch.einsum("td,tkdh->tkh", x.float(), keys.to(torch.bfloat16).float()[e])
     err = ((y.float() - ref)[~out_of_range].abs().max() / ref.abs().max()).item()
     assert err <= 2e-2
+
+
+@pytest.mark.parametrize("E", [1, 5, 16])
+@pytest.mark.parametrize("load", ["even", "one_long", "one_empty"])
+def test_weight_gradient_chunk_order(E, load):
+    # 400 routes per expert: chunks run longest first if some expert has more
+    # than 1.25 times the mean, else in expert order
+    g = torch.Generator().manual_seed(E)
+    T, K, D, H = 100 * E, 4, 136, 128
+    sel = (torch.arange(T * K) % E).view(T, K)
+    if load == "one_long":
+        sel[torch.rand(T, K, generator=g) < 0.5] = E - 1
+    elif load == "one_empty":
+        sel[sel == 0] = E // 2
+    x = torch.randn(T, D, generator=g).to(torch.bfloat16)
+    keys = torch.randn(E, D, H, generator=g) / D ** 0.5
+    go = torch.randn(T, K, H, generator=g).to(torch.bfloat16)
+    got = U.run_hip(x, keys, sel, None, go, False, True)
+    exp = U.run_oracle(x, keys, sel, None, go, False, True)
+    U.compare(got, exp, 2e-2)
