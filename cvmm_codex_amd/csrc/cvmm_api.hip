@@ -1007,8 +1007,10 @@ static int fwd_core(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld
   p.n_out = p.N;  // (padded columns are products of zeros)
   p.o_idx = nullptr;
   // route input kept for the weight gradient: the small-K kernel writes the
-  // scaled rows from its activation fragments (the rows cvmm_bwd_w scales)
-  const bool keep = scaled_rows != nullptr && scaled_written != nullptr && out_index == nullptr &&
+  // scaled rows from its activation fragments (the rows cvmm_bwd_w scales).
+  // Not from padded copies: the kernel's rows are p.K wide, the caller's d_in,
+  // and the weight gradient scales those rows as it pads them.
+  const bool keep = scaled_rows != nullptr && scaled_written != nullptr && out_index == nullptr && !pad_sizes &&
                     x_rows == n_routes && out_dtype == op_dtype && (op_dtype == kBF16 || op_dtype == kF16) &&
                     routed_gemm_is_panel(p, op_dtype);
   if (keep) {

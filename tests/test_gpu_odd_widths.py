@@ -38,6 +38,10 @@ def _run(T, K, D, H, E, weighted, route_input, xdt, kdt, op, hot):
     (700, 8, 136, 181),     # only d_out off the grid
     (700, 8, 181, 128),     # only d_in off the grid
     (400, 2, 523, 321),     # 256-wide weight-gradient tiles' range
+    (1400, 8, 100, 512),    # short-K forward whose padded output fills whole 64-column tiles (the kernel
+    (1400, 8, 60, 1024),    # that can keep scaled route rows: here p.K != d_in, none are kept)
+    (1400, 8, 126, 1020),
+    (1400, 8, 64, 1020),    # the same with only d_out off the grid
 ])
 @pytest.mark.parametrize("weighted,route_input", [(False, False), (True, True), (True, False), (False, True)])
 def test_padded_widths(T, K, D, H, weighted, route_input):
