@@ -217,19 +217,18 @@ __device__ bool gemm_schedule(const GemmParams& p, int64_t n_groups, RouteMeta<B
   return true;
 }
 
-// 16 bytes of a row (4 / 2-byte elements, `left` of them inside the row) at
-// any element alignment: one store where they all are.
-template <int ESZ>
-__device__ __forceinline__ void store_piece(char* dst, const uint32_t (&d)[4], int64_t left) {
-  if (left >= 16 / ESZ) {
+// 8 columns of a 16-bit row (`left` of them inside the row) at any element
+// alignment: one store where they all are.
+__device__ __forceinline__ void store_piece16(char* dst, const uint32_t (&d)[4], int64_t left) {
+  if (left >= 8) {
     __builtin_memcpy(dst, d, 16);
     return;
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    if (left >= (i + 1) * (4 / ESZ)) {
+    if (left >= 2 * (i + 1)) {
       __builtin_memcpy(dst + 4 * i, &d[i], 4);
-    } else if (ESZ == 2 && left == 2 * i + 1) {
+    } else if (left == 2 * i + 1) {
       const uint16_t h = (uint16_t)d[i];
       __builtin_memcpy(dst + 4 * i, &h, 2);
     }

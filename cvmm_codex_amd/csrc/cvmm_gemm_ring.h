@@ -352,17 +352,16 @@ __global__ __launch_bounds__(NW * 64, OCC) void routed_gemm_ring_kernel(const Ge
   // DG without a peeled last slice (the read-ahead loop): the x pieces now
   if constexpr (DG && RA) load_x();
   // one row piece of 4 x 16 columns: lane values -> 16-byte (or 4 x 16-byte
-  // fp32) stores of row rowp
-  auto store_row = [&](char* rowp, const float (&v)[4][4]) {
+  // fp32) stores of row rowp; `pieces`: rows of n_out < N columns (16-bit
+  // outputs only) at any alignment, element by element at their ends
+  auto store_row = [&](auto pieces, char* rowp, const float (&v)[4][4]) {
+    constexpr bool PIECES = decltype(pieces)::value;
     if constexpr (sizeof(OutT) == 4) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int64_t n = nwave + i * 16 + 4 * fq;
-        if (rowp != nullptr && n < p.n_out) {
-          const uint32_t d[4] = {__float_as_uint(v[i][0]), __float_as_uint(v[i][1]), __float_as_uint(v[i][2]),
-                                 __float_as_uint(v[i][3])};
-          store_piece<4>(rowp + n * 4, d, p.n_out - n);
-        }
+        if (rowp != nullptr && n < p.N)
+          *reinterpret_cast<float4*>(rowp + n * 4) = make_float4(v[i][0], v[i][1], v[i][2], v[i][3]);
       }
     } else {
       // blocks 2p, 2p+1 -> columns 32p + 8*fq + [0, 8) per lane (two lane swaps)
@@ -384,56 +383,68 @@ __global__ __launch_bounds__(NW * 64, OCC) void routed_gemm_ring_kernel(const Ge
         const auto t0 = __builtin_amdgcn_permlane16_swap(s0[0], s0[1], false, false);
         const auto t1 = __builtin_amdgcn_permlane16_swap(s1[0], s1[1], false, false);
         const int64_t n = nwave + pr * 32 + 8 * fq;
-        if (rowp != nullptr && n < p.n_out) {
+        if constexpr (PIECES) {
           const uint32_t d[4] = {t0[0], t1[0], t0[1], t1[1]};
-          store_piece<2>(rowp + n * 2, d, p.n_out - n);
+          if (rowp != nullptr && n < p.n_out) store_piece16(rowp + n * 2, d, p.n_out - n);
+        } else if (rowp != nullptr && n < p.N) {
+          *reinterpret_cast<uint4*>(rowp + n * 2) = make_uint4(t0[0], t1[0], t0[1], t1[1]);
         }
       }
     }
   };
+  auto store_rows = [&](auto pieces) {
 #pragma unroll
-  for (int j = 0; j < MB; ++j) {
-    const int m = wm * WR + j * 16 + fr;
-    const int64_t orow = meta.orow[m];
-    float v[4][4];
-    if (plain) {
+    for (int j = 0; j < MB; ++j) {
+      const int m = wm * WR + j * 16 + fr;
+      const int64_t orow = meta.orow[m];
+      float v[4][4];
+      if (plain) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[i][q] = acc[i][j][q];
-    } else {
-      const float wv = meta.w[m];
+          for (int q = 0; q < 4; ++q) v[i][q] = acc[i][j][q];
+      } else {
+        const float wv = meta.w[m];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          float c = round_to(acc[i][j][q], p.val_dtype);
-          if (has_w) {
-            c = c * wv;
-            if (p.prod_dtype >= 0) c = round_to(c, p.prod_dtype);
+          for (int q = 0; q < 4; ++q) {
+            float c = round_to(acc[i][j][q], p.val_dtype);
+            if (has_w) {
+              c = c * wv;
+              if (p.prod_dtype >= 0) c = round_to(c, p.prod_dtype);
+            }
+            v[i][q] = c;
           }
-          v[i][q] = c;
-        }
-    }
-    char* rowp = orow >= 0 ? reinterpret_cast<char*>(p.out) + orow * p.out_ld * (int64_t)sizeof(OutT) : nullptr;
-    if (p.act == 0) {
-      store_row(rowp, v);
-    } else {
-      // GELU: h = the product in the output type (kept for the backward),
-      // out = gelu(h) rounded to the output type
-      char* auxp = orow >= 0 ? reinterpret_cast<char*>(p.aux) + orow * p.out_ld * (int64_t)sizeof(OutT) : nullptr;
-      float y[4][4];
+      }
+      char* rowp = orow >= 0 ? reinterpret_cast<char*>(p.out) + orow * p.out_ld * (int64_t)sizeof(OutT) : nullptr;
+      if (Role != 0 || p.act == 0) {  // (the GELU comes with the forward only)
+        store_row(pieces, rowp, v);
+      } else {
+        // GELU: h = the product in the output type (kept for the backward),
+        // out = gelu(h) rounded to the output type
+        char* auxp = orow >= 0 ? reinterpret_cast<char*>(p.aux) + orow * p.out_ld * (int64_t)sizeof(OutT) : nullptr;
+        float y[4][4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float h = (float)(OutT)v[i][q];
-          v[i][q] = h;
-          y[i][q] = gelu_erf(h);
-        }
-      store_row(auxp, v);
-      store_row(rowp, y);
+          for (int q = 0; q < 4; ++q) {
+            const float h = (float)(OutT)v[i][q];
+            v[i][q] = h;
+            y[i][q] = gelu_erf(h);
+          }
+        store_row(pieces, auxp, v);
+        store_row(pieces, rowp, y);
+      }
     }
+  };
+  // (one test for all rows: with it inside the row loop the compiler makes 8-
+  // and 4-byte stores of the 16-byte ones)
+  if constexpr (sizeof(OutT) == 4) {
+    store_rows(std::false_type{});
+  } else {
+    if (p.n_out == p.N) store_rows(std::false_type{});
+    else store_rows(std::true_type{});
   }
 
   if constexpr (DG) {
@@ -516,8 +527,8 @@ inline bool ring_eligible(const GemmParams& p, int32_t op) {
                               (reinterpret_cast<uintptr_t>(p.dg_x) & 7) == 0 && p.dg_x_ld % 4 == 0)) &&
          (p.act == 0 || (p.aux != nullptr && (p.n_out < p.N || (reinterpret_cast<uintptr_t>(p.aux) % 16) == 0))) &&
          (p.out_dtype == op || p.out_dtype == kF32) && p.N % 8 == 0 &&
-         // (a padded N stores rows of n_out columns at any alignment)
-         (p.n_out < p.N || ((reinterpret_cast<uintptr_t>(p.out) % 16) == 0 && ((size_t)p.out_ld * esz) % 16 == 0));
+         // (a padded N stores rows of n_out 16-bit columns at any alignment)
+         (p.n_out == p.N || p.out_dtype == op) && (p.n_out < p.N || ((reinterpret_cast<uintptr_t>(p.out) % 16) == 0 && ((size_t)p.out_ld * esz) % 16 == 0));
 }
 
 template <typename OpT, typename OutT, int BM, int BN, int STAGES, int OCC, bool RA, int BK, bool BNC, int NW>
@@ -605,6 +616,10 @@ hipError_t launch_routed_gemm_ring_out(const GemmParams& p, hipStream_t stream) 
     return launch_routed_gemm_ring_t<OpT, OutT, 160, 128, 2, 2, false, 64>(p, stream);
   return launch_routed_gemm_ring_t<OpT, OutT, 128, 128, 2, 2, false, 64>(p, stream);
 }
+
+// The 16-bit outputs are compiled in units of their own (cvmm_gemm_ring_*.hip).
+extern template hipError_t launch_routed_gemm_ring_out<bf16_t, bf16_t>(const GemmParams&, hipStream_t);
+extern template hipError_t launch_routed_gemm_ring_out<f16_t, f16_t>(const GemmParams&, hipStream_t);
 
 // Fast-path dispatch for 16-bit k-contiguous operands: small K -> panel
 // kernel, long K -> ring kernel, anything else (routing-weight gradient,
