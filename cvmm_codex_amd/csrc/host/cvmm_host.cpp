@@ -386,8 +386,11 @@ Tensor cvmm_forward_impl(const Tensor& x, const Tensor& keys, const OptT& keys_o
   if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, opts(x, at::kByte));
   if (scaled != nullptr && rwf.has_value() && !oi.has_value() && xf.size(0) == R && outd == od &&
       (op == at::kBFloat16 || op == at::kHalf) && !(flags & CVMM_FLAG_ATOMIC_REDUCE) &&
-      (cvmm_topk_dense(out_rows, (int32_t)E, d_in, d_out, k, od) == 1 || d_in <= 128)) {
-    // (the dense sum, or a small-K routed product: the two that keep them)
+      (cvmm_topk_dense(out_rows, (int32_t)E, d_in, d_out, k, od) == 1 ||
+       (d_in <= 128 && d_in % 8 == 0 && d_out % 64 == 0 && kv.stride(1) == 1))) {
+    // (the dense sum, or a small-K routed product: the two that keep them.
+    // The latter reads the [E, d_out, d_in] copy and fills whole 64-column
+    // tiles; padded widths and weights read as stored keep none.)
     Tensor xs = at::empty({R, d_in}, opts(x, op));
     int32_t written = 0;
     check(cvmm_fwd_keep_scaled(ptr(xf), dtype_id(xf.scalar_type()), xf.size(0), xf.stride(0), ptr(kv),

@@ -92,3 +92,27 @@ def test_stored_weights_views_fall_back():
     ref = torch.stack([torch.stack([x[t].double() @ keys[sel[t, j]].double() for j in range(k)]) for t in range(T)])
     for o in outs:
         _check(o, ref)
+
+
+@pytest.mark.parametrize("T,k,E,D,H,weights", [
+    (60, 2, 16, 128, 256, "bf16"),    # few routes: the weights are read as they are stored
+    (400, 2, 16, 128, 200, "fp32"),   # an output of no whole 64-column tiles
+    (1400, 8, 7, 100, 512, "fp32")])  # padded copies
+def test_no_scaled_rows_are_made_where_none_are_kept(T, k, E, D, H, weights):
+    """A weighted route-input forward that trains the weights makes the
+    tensors of one that does not: no [R, d_in] rows that nothing fills."""
+    _, keys, sel = _case(T, k, E, D, H, "bf16", weights, False, D)
+    x = torch.randn(T, k, D, device="cuda").to(torch.bfloat16)
+    w = torch.rand(T, k, device="cuda")
+
+    def made(kv):
+        for _ in range(2):
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                s = C.cvmm_prepare_sel2(sel, w, route_input=True)
+                before = torch.cuda.memory_stats()["allocation.all.allocated"]
+                C.cvmm(x, s, kv)
+            n = torch.cuda.memory_stats()["allocation.all.allocated"] - before
+        return n
+
+    training, frozen = made(keys.clone().requires_grad_()), made(keys)
+    assert training == frozen
