@@ -114,6 +114,7 @@ _SIGS = {
     "cvmm_bwd_w_counter_bytes": (_SZ, [_I64, _I32, _I64, _I64, _I32]),
     "cvmm_bwd_w_workspace_bytes": (_SZ, [_I64, _I32, _I64, _I64, _I32, _I32]),
     "cvmm_bwd_w_workspace_bytes_ex": (_SZ, [_I64, _I32, _I64, _I64, _I32, _I32, _I32]),
+    "cvmm_bwd_w_rows_bytes": (_SZ, [_I64, _I64, _I64, _I32, _I64, _I64, _I32, _I32]),
     "cvmm_bwd_w": (ctypes.c_int, [
         _P, _I32, _I64, _I64,                 # x
         _P, _I32, _I64, _I64,                 # grad
@@ -122,6 +123,14 @@ _SIGS = {
         _P, _I32, _I64, _I32,                 # rw, rw dtype, top_k, op
         _P, _I32, _I64, _I64, _I64,           # grad_keys, dtype, strides
         _I32, _P, _SZ, _P]),
+    "cvmm_bwd_w_rows": (ctypes.c_int, [
+        _P, _I32, _I64, _I64,                 # x
+        _P, _I32, _I64, _I64,                 # grad
+        _I32, _I64, _I64,                     # E, d_in, d_out
+        _P, _P, _P, _I64, _P,                 # sorted_sel, sel_index, out_index, R, offsets
+        _P, _I32, _I64, _I32,                 # rw, rw dtype, top_k, op
+        _P, _I32, _I64, _I64, _I64,           # grad_keys, dtype, strides
+        _I32, _P, _SZ, _P, _SZ, _P]),         # flags, rows, workspace, stream
 }
 
 EXPORTED = tuple(_SIGS)

@@ -1359,22 +1359,34 @@ size_t cvmm_bwd_w_workspace_bytes(int64_t n_routes, int32_t n_experts, int64_t d
   return c.used;
 }
 
-size_t cvmm_bwd_w_workspace_bytes_ex(int64_t n_routes, int32_t n_experts, int64_t d_in, int64_t d_out,
-                                     int32_t op_dtype, int32_t has_offsets, int32_t weighted_route_input) {
-  size_t need = cvmm_bwd_w_workspace_bytes(n_routes, n_experts, d_in, d_out, op_dtype, has_offsets);
+size_t cvmm_bwd_w_rows_bytes(int64_t x_rows, int64_t grad_rows, int64_t n_routes, int32_t n_experts, int64_t d_in,
+                             int64_t d_out, int32_t op_dtype, int32_t weighted_route_input) {
+  if (x_rows <= 0 || grad_rows <= 0 || x_rows > n_routes || grad_rows > n_routes) return 0;
   if (pads_operands(op_dtype, n_routes, n_experts, d_in, d_out))  // padded x and gradient rows
-    return align_up(need, 256) + align_up((size_t)n_routes * pad8(d_in) * 2, 256) + (size_t)n_routes * pad8(d_out) * 2;
-  if (weighted_route_input && wgrad_scales_rows(op_dtype, d_in))
-    need = align_up(need, 256) + (size_t)n_routes * d_in * dtype_size(op_dtype);
-  return need;
+    return align_up((size_t)x_rows * pad8(d_in) * 2, 256) + (size_t)grad_rows * pad8(d_out) * 2;
+  if (weighted_route_input && wgrad_scales_rows(op_dtype, d_in)) return (size_t)x_rows * d_in * dtype_size(op_dtype);
+  return 0;
 }
 
-int cvmm_bwd_w(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld, const void* grad, int32_t grad_dtype,
-               int64_t grad_rows, int64_t grad_ld, int32_t n_experts, int64_t d_in, int64_t d_out,
-               const int32_t* sorted_sel, const int64_t* sel_index, const int64_t* out_index, int64_t n_routes,
-               const int64_t* offsets, const void* rw, int32_t rw_dtype, int64_t top_k, int32_t op_dtype,
-               void* grad_keys, int32_t grad_keys_dtype, int64_t gk_se, int64_t gk_si, int64_t gk_sj, int32_t flags,
-               void* workspace, size_t workspace_bytes, void* stream) {
+size_t cvmm_bwd_w_workspace_bytes_ex(int64_t n_routes, int32_t n_experts, int64_t d_in, int64_t d_out,
+                                     int32_t op_dtype, int32_t has_offsets, int32_t weighted_route_input) {
+  const size_t need = cvmm_bwd_w_workspace_bytes(n_routes, n_experts, d_in, d_out, op_dtype, has_offsets);
+  const size_t rows = cvmm_bwd_w_rows_bytes(n_routes, n_routes, n_routes, n_experts, d_in, d_out, op_dtype,
+                                            weighted_route_input);
+  return rows > 0 ? align_up(need, 256) + rows : need;
+}
+
+}  // extern "C"
+
+// cvmm_bwd_w; `rows` (or NULL): where the padded or scaled rows go, else
+// behind the workspace's partials where it has the room.
+static int bwd_w_core(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld, const void* grad,
+                      int32_t grad_dtype, int64_t grad_rows, int64_t grad_ld, int32_t n_experts, int64_t d_in,
+                      int64_t d_out, const int32_t* sorted_sel, const int64_t* sel_index, const int64_t* out_index,
+                      int64_t n_routes, const int64_t* offsets, const void* rw, int32_t rw_dtype, int64_t top_k,
+                      int32_t op_dtype, void* grad_keys, int32_t grad_keys_dtype, int64_t gk_se, int64_t gk_si,
+                      int64_t gk_sj, int32_t flags, void* rows, size_t rows_bytes, void* workspace,
+                      size_t workspace_bytes, void* stream) {
   const bool weighted = rw != nullptr;
   if (!valid_dtype(x_dtype) || !valid_dtype(grad_dtype) || !valid_dtype(op_dtype) || !valid_dtype(grad_keys_dtype) ||
       (weighted && !valid_dtype(rw_dtype)))
@@ -1425,24 +1437,25 @@ int cvmm_bwd_w(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld, con
   p.partial = (float*)c.take((size_t)p.max_slots * wgrad_partial_elems(d_in, d_out) * 4);
 
   const int64_t* rp = out_index ? out_index : sel_index;
-  // A weighted selection with route input (x row = route) whose workspace
-  // holds the rows: x scaled by its routes' weights once, rnd_op(rnd_op(w_r)
-  // * rnd_op(x_r)), then the unweighted kernel with the token's gradient row
-  // (the weight moves from the d_out-wide gradient slices of every dW tile to
-  // one pass over the d_in-wide route rows).
-  const size_t rows_bytes = (size_t)x_rows * d_in * dtype_size(op_dtype);
-  // Widths off the 16-byte grid, where the workspace holds the padded copies
-  // (the x rows of a weighted route-input selection scaled on the way).
-  const bool padded = pads_operands(op_dtype, n_routes, n_experts, d_in, d_out) && !rows_scaled && x_rows <= n_routes &&
-                      grad_rows <= n_routes &&
-                      align_up(c.used, 256) + align_up((size_t)n_routes * pad8(d_in) * 2, 256) +
-                              (size_t)n_routes * pad8(d_out) * 2 <= workspace_bytes;
-  const bool scale_rows = !padded && !rows_scaled && weighted && out_index == nullptr && x_rows <= n_routes && n_routes > 0 &&
-                          wgrad_scales_rows(op_dtype, d_in) && align_up(c.used, 256) + rows_bytes <= workspace_bytes;
+  // A weighted selection with route input (x row = route): x scaled by its
+  // routes' weights once, rnd_op(rnd_op(w_r) * rnd_op(x_r)), then the
+  // unweighted kernel with the token's gradient row (the weight moves from the
+  // d_out-wide gradient slices of every dW tile to one pass over the d_in-wide
+  // route rows).  Widths off the 16-byte grid: padded copies of both operands
+  // (such x rows scaled on the way).  Either where there is room for the rows.
+  const bool scaled = weighted && out_index == nullptr && !rows_scaled;
+  const size_t rows_need = rows_scaled ? 0 : cvmm_bwd_w_rows_bytes(x_rows, grad_rows, n_routes, n_experts, d_in, d_out,
+                                                                   op_dtype, scaled ? 1 : 0);
+  if (rows == nullptr) {
+    const size_t at = align_up(c.used, 256);
+    rows = (char*)workspace + at;
+    rows_bytes = workspace_bytes > at ? workspace_bytes - at : 0;
+  }
+  const bool room = rows_need > 0 && rows_need <= rows_bytes;
+  const bool padded = room && pads_operands(op_dtype, n_routes, n_experts, d_in, d_out);
   if (padded) {
-    const bool scaled = weighted && out_index == nullptr;
-    void* xp = c.take((size_t)n_routes * pad8(d_in) * 2);
-    void* gp = c.take((size_t)n_routes * pad8(d_out) * 2);
+    void* xp = rows;
+    void* gp = (char*)rows + align_up((size_t)x_rows * pad8(d_in) * 2, 256);
     int r = check_launch(timed_combine(s, [&] {
       return launch_pad_rows(x, x_dtype, x_ld, x_rows, d_in, scaled ? rw : nullptr, rw_dtype, op_dtype, xp, s);
     }), "cvmm_bwd_w(pad x)");
@@ -1457,16 +1470,15 @@ int cvmm_bwd_w(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld, con
     p.padded = 1;
   } else if (rows_scaled) {
     rw = nullptr;  // (the selection stays weighted: one gradient row per token)
-  } else if (scale_rows) {
-    void* xs = c.take(rows_bytes);
+  } else if (room) {
     // timed with the row work (combine class): the weight-gradient class
     // times the GEMM alone, one launch per call
     int r = check_launch(timed_combine(s, [&] {
-      return launch_scale_rows(x, x_dtype, x_ld, true, rw, rw_dtype, op_dtype, x_rows, top_k, d_in, op_dtype, xs,
+      return launch_scale_rows(x, x_dtype, x_ld, true, rw, rw_dtype, op_dtype, x_rows, top_k, d_in, op_dtype, rows,
                                s);
     }), "cvmm_bwd_w(scale)");
     if (r) return r;
-    x = xs;
+    x = rows;
     x_dtype = op_dtype;
     x_ld = d_in;
     rw = nullptr;
@@ -1506,6 +1518,33 @@ int cvmm_bwd_w(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld, con
     p.order = order == 1 ? kWgOrderChunk : order == 3 ? kWgOrderChunkXcd : kWgOrderTile;
   }
   return check_launch(timed(CVMM_KC_WGRAD, s, [&] { return launch_wgrad(p, op_dtype, s); }), "cvmm_bwd_w(gemm)");
+}
+
+extern "C" {
+
+int cvmm_bwd_w(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld, const void* grad, int32_t grad_dtype,
+               int64_t grad_rows, int64_t grad_ld, int32_t n_experts, int64_t d_in, int64_t d_out,
+               const int32_t* sorted_sel, const int64_t* sel_index, const int64_t* out_index, int64_t n_routes,
+               const int64_t* offsets, const void* rw, int32_t rw_dtype, int64_t top_k, int32_t op_dtype,
+               void* grad_keys, int32_t grad_keys_dtype, int64_t gk_se, int64_t gk_si, int64_t gk_sj, int32_t flags,
+               void* workspace, size_t workspace_bytes, void* stream) {
+  return bwd_w_core(x, x_dtype, x_rows, x_ld, grad, grad_dtype, grad_rows, grad_ld, n_experts, d_in, d_out, sorted_sel,
+                    sel_index, out_index, n_routes, offsets, rw, rw_dtype, top_k, op_dtype, grad_keys,
+                    grad_keys_dtype, gk_se, gk_si, gk_sj, flags, nullptr, 0, workspace, workspace_bytes,
+                    stream);
+}
+
+int cvmm_bwd_w_rows(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld, const void* grad, int32_t grad_dtype,
+                    int64_t grad_rows, int64_t grad_ld, int32_t n_experts, int64_t d_in, int64_t d_out,
+                    const int32_t* sorted_sel, const int64_t* sel_index, const int64_t* out_index, int64_t n_routes,
+                    const int64_t* offsets, const void* rw, int32_t rw_dtype, int64_t top_k, int32_t op_dtype,
+                    void* grad_keys, int32_t grad_keys_dtype, int64_t gk_se, int64_t gk_si, int64_t gk_sj, int32_t flags,
+                    void* rows, size_t rows_bytes, void* workspace, size_t workspace_bytes, void* stream) {
+  if (!aligned16(rows)) return fail(CVMM_ERR_INVALID, "cvmm_bwd_w_rows: rows not 16-byte aligned");
+  return bwd_w_core(x, x_dtype, x_rows, x_ld, grad, grad_dtype, grad_rows, grad_ld, n_experts, d_in, d_out, sorted_sel,
+                    sel_index, out_index, n_routes, offsets, rw, rw_dtype, top_k, op_dtype, grad_keys,
+                    grad_keys_dtype, gk_se, gk_si, gk_sj, flags, rows, rows_bytes, workspace, workspace_bytes,
+                    stream);
 }
 
 }  // extern "C"

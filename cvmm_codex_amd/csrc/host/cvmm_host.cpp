@@ -588,6 +588,10 @@ std::tuple<OptT, OptT, OptT> cvmm_backward_impl(const Tensor& grad_output, const
   // the weight gradient's x rows: declared before the join below, so that
   // a temporary (x converted to the op dtype) outlives the side stream's use
   Tensor xs;
+  // its copies of operand rows: allocated on the caller's stream before the
+  // fork and freed there after the join, like xs, and not kept (they are as
+  // large as the operands)
+  OptT rows;
   // joins the side stream back into `stream` on every way out below (and,
   // destroyed before the tensors declared above, before they are freed)
   SideJoin join;
@@ -597,9 +601,16 @@ std::tuple<OptT, OptT, OptT> cvmm_backward_impl(const Tensor& grad_output, const
     const bool pre_scaled = scaled_x.has_value();
     xs = pre_scaled ? *scaled_x : rows_of(fast && x.scalar_type() != op ? x.to(op) : storage_for(x, op), d_in);
     grad_w = at::empty(keys.sizes(), opts(keys, keys.scalar_type()));
+    // room for the scaled route rows of a weighted route-input selection
+    // (none when the forward kept them) or the padded rows of odd widths
+    const size_t rows_bytes =
+        pre_scaled ? 0
+                   : cvmm_bwd_w_rows_bytes(xs.size(0), g.size(0), R, (int32_t)E, d_in, d_out, od,
+                                           rw.has_value() && !oi.has_value() ? 1 : 0);
+    if (rows_bytes) rows = at::empty({(int64_t)rows_bytes}, opts(x, at::kByte));
     // with a grad-input to run as well, the weight gradient goes to the side
-    // stream once its inputs are enqueued; its inputs (g, xs and the routing
-    // tensors, all declared before `join`) are freed to the caller's stream
+    // stream once its inputs are enqueued; its inputs (g, xs, rows and the
+    // routing tensors, all declared before `join`) are freed to the caller's stream
     // only after the join, so no later work there reuses them too early
     int64_t wstream = stream;
     if ((flags & kHostOverlapBackward) && (need_grad_x || need_grad_rw)) {
@@ -607,10 +618,7 @@ std::tuple<OptT, OptT, OptT> cvmm_backward_impl(const Tensor& grad_output, const
       join.dev = x.get_device();
       join.main = (hipStream_t)(uintptr_t)stream;
     }
-    // a weighted route-input selection gets room for its scaled route rows
-    // (none needed when the forward kept them)
-    const size_t ws_bytes = cvmm_bwd_w_workspace_bytes_ex(R, (int32_t)E, d_in, d_out, od, 1,
-                                                          rw.has_value() && !oi.has_value() && !pre_scaled ? 1 : 0);
+    const size_t ws_bytes = cvmm_bwd_w_workspace_bytes(R, (int32_t)E, d_in, d_out, od, 1);
     const size_t ctr_bytes = cvmm_bwd_w_counter_bytes(R, (int32_t)E, d_in, d_out, od);
     Tensor ws;
     bool zeroed;
@@ -626,11 +634,12 @@ std::tuple<OptT, OptT, OptT> cvmm_backward_impl(const Tensor& grad_output, const
     }
     const int32_t wflags = (int32_t)flags | (zeroed ? CVMM_FLAG_COUNTERS_ZEROED : 0) |
                            (pre_scaled ? CVMM_FLAG_ROWS_SCALED : 0);
-    check(cvmm_bwd_w(ptr(xs), dtype_id(xs.scalar_type()), xs.size(0), xs.stride(0), ptr(g),
-                     dtype_id(g.scalar_type()), g.size(0), g.stride(0), (int32_t)E, d_in, d_out, tptr<int32_t>(s32),
-                     tptr<int64_t>(si), tptr<int64_t>(oi), R, tptr<int64_t>(offsets), ptr(rwf), rwd, k, od,
-                     ptr(grad_w), dtype_id(grad_w->scalar_type()), grad_w->stride(0), grad_w->stride(1),
-                     grad_w->stride(2), wflags, ptr(ws), (size_t)ws.numel(), (void*)wstream),
+    check(cvmm_bwd_w_rows(ptr(xs), dtype_id(xs.scalar_type()), xs.size(0), xs.stride(0), ptr(g),
+                          dtype_id(g.scalar_type()), g.size(0), g.stride(0), (int32_t)E, d_in, d_out,
+                          tptr<int32_t>(s32), tptr<int64_t>(si), tptr<int64_t>(oi), R, tptr<int64_t>(offsets),
+                          ptr(rwf), rwd, k, od, ptr(grad_w), dtype_id(grad_w->scalar_type()), grad_w->stride(0),
+                          grad_w->stride(1), grad_w->stride(2), wflags, ptr(rows), rows_bytes, ptr(ws),
+                          (size_t)ws.numel(), (void*)wstream),
           "cvmm_bwd_w");
   }
 

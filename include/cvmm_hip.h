@@ -444,15 +444,21 @@ size_t cvmm_bwd_w_counter_bytes(int64_t n_routes, int32_t n_experts, int64_t d_i
                                 int32_t op_dtype);
 size_t cvmm_bwd_w_workspace_bytes(int64_t n_routes, int32_t n_experts, int64_t d_in, int64_t d_out,
                                   int32_t op_dtype, int32_t has_offsets);
-/* The workspace of a weighted selection with route input (x row = route,
- * out_index NULL) given room for its scaled rows: with at least this many
- * bytes, cvmm_bwd_w scales each route row once, x'_r = rnd_op(rnd_op(w_r) *
+/* Bytes of the operand rows cvmm_bwd_w copies where it is given room for them
+ * (0: none).  A weighted selection with route input (x row = route, out_index
+ * NULL) has each route row scaled once, x'_r = rnd_op(rnd_op(w_r) *
  * rnd_op(x_r)) (16-bit op, d_in % 8 == 0), and runs the unweighted product
  * sum_i x'_i^T rnd_op(grad[rp(i)/top_k]) -- the weight applied to the route
  * row instead of the gradient row (the rounding point moves; the product is
- * the same).  With cvmm_bwd_w_workspace_bytes' size the weight is applied to
- * the gradient rows inside the kernel.  weighted_route_input = 0: the same as
- * cvmm_bwd_w_workspace_bytes.  No counterpart in the reference. */
+ * the same).  Widths that are not multiples of 8 (16-bit op, large enough)
+ * have both operands' rows padded with zeros, such x rows scaled on the way.
+ * Without the room the weight is applied to the gradient rows inside the
+ * kernel, and such widths run the general one.  No counterpart in the
+ * reference. */
+size_t cvmm_bwd_w_rows_bytes(int64_t x_rows, int64_t grad_rows, int64_t n_routes, int32_t n_experts, int64_t d_in,
+                             int64_t d_out, int32_t op_dtype, int32_t weighted_route_input);
+/* cvmm_bwd_w_workspace_bytes with room for those rows behind the rest (up to
+ * n_routes rows of each operand). */
 size_t cvmm_bwd_w_workspace_bytes_ex(int64_t n_routes, int32_t n_experts, int64_t d_in, int64_t d_out,
                                      int32_t op_dtype, int32_t has_offsets, int32_t weighted_route_input);
 int cvmm_bwd_w(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld,
@@ -462,6 +468,17 @@ int cvmm_bwd_w(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld,
                const int64_t* offsets, const void* reduction_weight, int32_t rw_dtype, int64_t top_k,
                int32_t op_dtype, void* grad_keys, int32_t grad_keys_dtype, int64_t gk_se, int64_t gk_si,
                int64_t gk_sj, int32_t flags, void* workspace, size_t workspace_bytes, void* stream);
+/* cvmm_bwd_w with the row copies in a buffer of their own (`rows`, 16-byte
+ * aligned, or NULL): a caller that keeps the workspace for its counters need
+ * not keep rows as large as the operands with it. */
+int cvmm_bwd_w_rows(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld,
+                    const void* grad, int32_t grad_dtype, int64_t grad_rows, int64_t grad_ld,
+                    int32_t n_experts, int64_t d_in, int64_t d_out,
+                    const int32_t* sorted_sel, const int64_t* sel_index, const int64_t* out_index, int64_t n_routes,
+                    const int64_t* offsets, const void* reduction_weight, int32_t rw_dtype, int64_t top_k,
+                    int32_t op_dtype, void* grad_keys, int32_t grad_keys_dtype, int64_t gk_se, int64_t gk_si,
+                    int64_t gk_sj, int32_t flags, void* rows, size_t rows_bytes, void* workspace,
+                    size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

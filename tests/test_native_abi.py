@@ -72,6 +72,24 @@ def test_workspace_queries(lib):
         lib.cvmm_bwd_w_workspace_bytes(65536, 64, 128, 1024, N.F32, 1)
 
 
+def test_row_copy_queries(lib):
+    """cvmm_bwd_w's row copies by the rows there are; the one-workspace query
+    has room for up to n_routes of each."""
+    rows = lib.cvmm_bwd_w_rows_bytes
+    # weighted route input: the scaled rows; none unweighted, in fp32, or for rows past the routes
+    assert rows(65536, 8192, 65536, 64, 128, 1024, N.BF16, 1) == 65536 * 128 * 2
+    assert rows(65536, 8192, 65536, 64, 128, 1024, N.BF16, 0) == 0
+    assert rows(65536, 8192, 65536, 64, 128, 1024, N.F32, 1) == 0
+    assert rows(65537, 8192, 65536, 64, 128, 1024, N.BF16, 1) == 0
+    # padded widths: both operands' rows (412 -> 416, 130 -> 136 columns), token or route input
+    for x_rows, g_rows in ((4095, 32760), (32760, 4095), (32760, 32760)):
+        need = (x_rows * 416 * 2 + 255) // 256 * 256 + g_rows * 136 * 2
+        assert rows(x_rows, g_rows, 32760, 63, 412, 130, N.BF16, 0) == need
+        assert rows(x_rows, g_rows, 32760, 63, 412, 130, N.BF16, 1) == need
+    base = lib.cvmm_bwd_w_workspace_bytes(32760, 63, 412, 130, N.BF16, 1)
+    assert lib.cvmm_bwd_w_workspace_bytes_ex(32760, 63, 412, 130, N.BF16, 1, 0) >= base + need
+
+
 def test_invalid_arguments_fail_before_launch(lib):
     rc = lib.cvmm_sort_routes(None, 0, 10, 0, 1, None, None, None, None, None, None, None, 0, None)
     assert rc == 1 and b"n_experts" in lib.cvmm_last_error()
