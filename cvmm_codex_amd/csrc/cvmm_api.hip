@@ -1513,7 +1513,8 @@ static int bwd_w_core(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_
     int bm, bn;
     wgrad_fast_tile(d_in, d_out, p.tile_choice, &bm, &bn);
     const bool even = (bm == 128 && bn == 128) || (bm == 256 && bn == 256);
-    p.order = wgrad_fast_eligible(p, op_dtype) && even ? kWgOrderChunkXcd : kWgOrderTile;
+    if (op_dtype == kF32) p.order = f32_wgrad_order(n_experts);
+    else p.order = wgrad_fast_eligible(p, op_dtype) && even ? kWgOrderChunkXcd : kWgOrderTile;
   } else {
     p.order = order == 1 ? kWgOrderChunk : order == 3 ? kWgOrderChunkXcd : kWgOrderTile;
   }

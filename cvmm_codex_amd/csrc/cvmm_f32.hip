@@ -337,7 +337,12 @@ __global__ __launch_bounds__(kGemmThreads, (F32WgCfg<BM, BN>::OCC)) void wgrad_f
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t tiles_n = (p.N + BN - 1) / BN, tiles = ((p.M + BM - 1) / BM) * tiles_n;
   int64_t slot_id, tile;  // (grid = round_up(chunks, 8) * tiles)
-  wgrad_chunk_xcd(blockIdx.x, (uint32_t)tiles, &slot_id, &tile);
+  if (p.order == kWgOrderChunkXcd) {
+    wgrad_chunk_xcd(blockIdx.x, (uint32_t)tiles, &slot_id, &tile);
+  } else {
+    slot_id = blockIdx.x / (uint32_t)tiles;
+    tile = blockIdx.x - (uint32_t)slot_id * (uint32_t)tiles;
+  }
   const int64_t m0 = (tile / tiles_n) * BM, n0 = (tile % tiles_n) * BN;
   if (!wgrad_schedule<kGemmThreads>(p, slot_id, sc, reinterpret_cast<int32_t*>(ring), true)) return;
   const int32_t expert = uniform_i32(sc.expert);
@@ -563,6 +568,15 @@ void f32_wgrad_tile(int64_t M, int64_t N, int32_t n_experts, int* bm, int* bn) {
   *bn = N <= 64 ? 64 : 128;
   *bm = M <= 64 ? 64 : (wide || N <= 64) ? 128 : 64;
 }
+
+// Workgroup order: a slot's tiles one after another over all XCDs, or from 64
+// experts the slots dealt to the XCDs (the tiles of a slot share its rows in
+// one L2).  Fewer slots leave XCDs idle or uneven when dealt: 1024 x 1024, 720
+// routes, spread / dealt, evenly loaded and by Zipf's law: 2 experts 27 / 74
+// and 33 / 89 us, 9: 34 / 48 and 33 / 62, 32: 45 / 46 and 49 / 68, 64: 86 / 84
+// and 86 / 98; 1024 x 128, 16384 routes: 48 experts 58 / 57 and 67 / 68, 64:
+// 56 / 54 and 71 / 71.
+int32_t f32_wgrad_order(int32_t n_experts) { return n_experts >= 64 ? kWgOrderChunkXcd : kWgOrderChunk; }
 
 hipError_t launch_f32_wgrad(const WgradParams& p, hipStream_t stream) {
   int bm, bn;

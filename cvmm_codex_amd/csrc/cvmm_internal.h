@@ -197,6 +197,7 @@ int64_t wgrad_partial_elems(int64_t M, int64_t N);
 int32_t wgrad_auto_tile(int64_t M, int64_t N, int64_t n_routes, int32_t n_experts);
 // the fp32 kernel's dW tile (cvmm_f32.hip)
 void f32_wgrad_tile(int64_t M, int64_t N, int32_t n_experts, int* bm, int* bn);
+int32_t f32_wgrad_order(int32_t n_experts);
 
 // ---------------------------------------------------------------------------
 // selector preparation

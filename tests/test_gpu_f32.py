@@ -52,10 +52,51 @@ def test_f32_split_weight_gradient(D, H):
     lib = N.lib()
     assert lib.cvmm_tuning_set(N.TUNE_WGRAD_CHUNK, 256) == 0
     try:
-        _run(700, 4, D, H, 4, False, False, hot=True)
+        _run(max(700, 26_000_000 // (D * H)), 4, D, H, 4, False, False, hot=True)  # (>= 1e8 products)
         _run(700, 4, D, H, 4, True, False, hot=True)
     finally:
         lib.cvmm_tuning_set(N.TUNE_WGRAD_CHUNK, 0)
+
+
+@pytest.mark.parametrize("chunk", [0, 32])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_f32_weight_gradient_of_128_wide_tiles(weighted, chunk):
+    """Eight 128 x 128 tiles per CU (512 experts of 256 x 256), whole experts
+    and experts in chunks of 32 routes."""
+    lib = N.lib()
+    assert lib.cvmm_tuning_set(N.TUNE_WGRAD_CHUNK, chunk) == 0
+    try:
+        _run(500, 4, 256, 256, 512, weighted, weighted, hot=True)
+    finally:
+        lib.cvmm_tuning_set(N.TUNE_WGRAD_CHUNK, 0)
+
+
+@pytest.mark.parametrize("E,R,D,H", [(1, 720, 512, 512), (2, 4096, 512, 256), (5, 4096, 132, 260), (9, 720, 512, 512),
+                                     (63, 8192, 132, 132), (64, 8192, 132, 132)])
+def test_f32_weight_gradient_orders(E, R, D, H):
+    """Below 64 experts the tiles of a chunk spread over the XCDs, from there
+    chunks are dealt to them; few routes per expert are split from 256 on.
+    Both orders' bits are the same, and the built-in one's."""
+    g = torch.Generator().manual_seed(E)
+    x = torch.randn(R // 4, D, generator=g).cuda()
+    keys = torch.randn(E, D, H, generator=g).cuda().requires_grad_()
+    p = torch.arange(1, E + 1.).pow(-0.7)
+    ids = torch.multinomial(p, R, replacement=True, generator=g).view(-1, 4).cuda()
+    go = torch.randn(R // 4, 4, H, generator=g).cuda()
+    lib = N.lib()
+    y = C.cvmm(x, C.cvmm_prepare_sel2(ids), keys)
+    out = []
+    try:
+        for order in (0, 1, 3):
+            assert lib.cvmm_tuning_set(N.TUNE_WGRAD_ORDER, order) == 0
+            out.append(torch.autograd.grad(y, keys, go, retain_graph=True)[0])
+    finally:
+        lib.cvmm_tuning_set(N.TUNE_WGRAD_ORDER, 0)
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+    rows = x.double().repeat_interleave(4, 0)
+    flat, gd = ids.reshape(-1), go.double().reshape(R, H)
+    ref = torch.stack([rows[flat == e].T @ gd[flat == e] for e in range(E)])
+    assert ((out[0].double() - ref).abs().max() / ref.abs().max()).item() <= 1e-5
 
 
 def test_f32_transposed_keys_and_unrouted_ids():
