@@ -344,7 +344,9 @@ __global__ __launch_bounds__(kGemmThreads, (F32WgCfg<BM, BN>::OCC)) void wgrad_f
     tile = blockIdx.x - (uint32_t)slot_id * (uint32_t)tiles;
   }
   const int64_t m0 = (tile / tiles_n) * BM, n0 = (tile % tiles_n) * BN;
-  if (!wgrad_schedule<kGemmThreads>(p, slot_id, sc, reinterpret_cast<int32_t*>(ring), true)) return;
+  if (!wgrad_schedule<kGemmThreads>(p, slot_id, sc, reinterpret_cast<int32_t*>(ring),
+                                   kWgSortRoutes32))
+    return;
   const int32_t expert = uniform_i32(sc.expert);
   const int64_t lo = sc.lo, hi = sc.hi;
   const int32_t nch = uniform_i32(sc.nch);

@@ -13,9 +13,11 @@ struct WgSched {
 };
 
 // Experts the sorted order is computed for (one per thread), and the mean
-// routes per expert from which it is.
+// routes per expert from which it is: 16-bit kernels, fp32 ones, none.
 constexpr int32_t kWgSortExperts = 256;
-constexpr int64_t kWgSortRoutes = 384;
+constexpr int64_t kWgSortRoutes16 = 768, kWgSortRoutes32 = 384, kWgNoSort = int64_t(1) << 40;
+constexpr int kWgSchedScratch = 2 * kWgSortExperts + 4;
+static_assert(kWgSortExperts == 4 * 64, "four flags");
 
 // (expert, route chunk) of work slot `slot_id`.  An expert of n routes is cut
 // into ceil(n / p.split) chunks of equal length (multiples of 32 routes; at
@@ -23,17 +25,22 @@ constexpr int64_t kWgSortRoutes = 384;
 // longest first (ties by id), so that the long chunks start first and the
 // short ones fill the end of the launch: a router's loads differ by 2x and
 // more between experts, and in id order the launch ended on whichever expert
-// came last.  More than kWgSortExperts experts keep id order, and so do
-// launches of few routes per expert, where the order costs every workgroup
-// more than it evens out (18 routes on each of 122 experts: 38 us against 29
-// per launch; 330 on each of 40, evenly loaded: 16.1 against 14.7) and those where no expert has more than
-// 1.25 times the mean (1024 routes on each of 64, 1024 x 128: 38.2 us sorted,
-// 36.0 by this test, 34.8 with no test).  Every workgroup computes the same
-// order; `scratch` is 2 * kWgSortExperts ints of LDS, free again when this returns.  Returns false (uniformly) past the last
-// slot.
+// came last (64 experts of 1024 x 128, 1024 routes each, loads up to 1.4 times
+// that: 42 us per launch in id order, 40 sorted).  Id order stays
+//  - for more than kWgSortExperts experts, and up to 8 (they are dealt to one
+//    XCD each: 8 of 1024 x 4096, loads up to 1.4 times the mean, 182 us
+//    sorted, 172 not);
+//  - below `sort_routes` routes per expert, where ranking costs every
+//    workgroup what it evens out: 512 of them on each of 16, 2048 x 512, 44.3
+//    us sorted, 42.6 not; 18 on each of 122 experts 38 and 29;
+//  - where no expert has more than 1.25 times the mean (1024 routes on each of
+//    64, 1024 x 128: 38.2 us sorted; 34.5 by this test, as without it).
+// Every workgroup computes the same order.  `scratch` is kWgSchedScratch ints
+// of LDS, 16-byte aligned, free again when this returns.  Returns false
+// (uniformly) past the last slot.
 template <int NT>
 __device__ __forceinline__ bool wgrad_schedule(const WgradParams& p, int64_t slot_id, WgSched& s, int32_t* scratch,
-                                               bool by_length) {
+                                               int64_t sort_routes) {
   static_assert(NT >= kWgSortExperts, "one thread per sorted expert");
   const int tid = threadIdx.x, lane = tid & 63;
   auto range = [&](int32_t e, int64_t& st, int64_t& n) {
@@ -46,24 +53,29 @@ __device__ __forceinline__ bool wgrad_schedule(const WgradParams& p, int64_t slo
       n = end > start ? end - start : 0;
     }
   };
+  // (most launches split no expert: no division there)
   auto chunks_of = [&](int32_t e, int64_t n) -> int32_t {
     if (e >= p.n_experts) return 0;
-    const int64_t c = (n + p.split - 1) / p.split;
-    return c < 1 ? 1 : (int32_t)c;
+    return n <= p.split ? 1 : (int32_t)((n + p.split - 1) / p.split);
   };
-  bool sorted = by_length && p.n_experts <= kWgSortExperts && p.n_routes >= kWgSortRoutes * p.n_experts;
+  auto chunk_len = [](int64_t n, int32_t nch) -> int64_t { return nch == 1 ? n : (n + nch - 1) / nch; };
+  bool sorted = p.n_experts <= kWgSortExperts && p.n_experts > 8 && p.n_routes >= sort_routes * p.n_experts;
   int32_t* len = scratch;                    // chunk length of expert e
   int32_t* order = scratch + kWgSortExperts; // expert of rank r
+  int32_t* flags = order + kWgSortExperts;   // whether a wave's experts are uneven
+  // this thread's expert; wave 0's are the scan's first 64 in id order
+  int64_t st0 = 0, n0 = 0;
+  if (tid < 64 || sorted) range(tid, st0, n0);
   if (sorted) {
-    int32_t uneven = 0;
     if (tid < kWgSortExperts) {
-      int64_t st, n;
-      range(tid, st, n);
-      const int32_t nch = chunks_of(tid, n);
-      len[tid] = nch > 0 ? (int32_t)((n + nch - 1) / nch) : -1;
-      uneven = 4 * n * p.n_experts > 5 * p.n_routes;
+      const int32_t nch = chunks_of(tid, n0);
+      len[tid] = nch > 0 ? (int32_t)chunk_len(n0, nch) : -1;
+      const bool uneven = __any(4 * n0 * p.n_experts > 5 * p.n_routes);
+      if (lane == 0) flags[tid >> 6] = uneven;
     }
-    sorted = __syncthreads_or(uneven) != 0;  // (a barrier: len is written)
+    __syncthreads();
+    const int4 f = *reinterpret_cast<const int4*>(flags);
+    sorted = (f.x | f.y | f.z | f.w) != 0;
     if (sorted && tid < p.n_experts) {
       const int32_t mine = len[tid];
       int32_t rank = 0;
@@ -90,15 +102,15 @@ __device__ __forceinline__ bool wgrad_schedule(const WgradParams& p, int64_t slo
     for (int32_t base = 0; base < p.n_experts; base += 64) {
       const int32_t r = base + lane;
       const int32_t e = r < p.n_experts ? (sorted ? order[r] : r) : p.n_experts;
-      int64_t st, n;
-      range(e, st, n);
+      int64_t st = st0, n = n0;
+      if (sorted || base > 0) range(e, st, n);
       const int32_t nch = chunks_of(e, n);
       const int32_t multi = nch > 1 ? nch : 0;
       const int32_t incl = wave_incl_scan(nch) + carry, incl_m = wave_incl_scan(multi) + carry_multi;
       const int32_t excl = incl - nch;
       if (nch > 0 && slot_id >= excl && slot_id < incl) {
         const int64_t c = slot_id - excl;
-        const int64_t step = ((n + nch - 1) / nch + 31) / 32 * 32;
+        const int64_t step = (chunk_len(n, nch) + 31) / 32 * 32;
         const int64_t a = c * step < n ? c * step : n, b = (c + 1) * step < n && c + 1 < nch ? (c + 1) * step : n;
         s.expert = e;
         s.nch = nch;

@@ -138,7 +138,7 @@ __global__ __launch_bounds__(WM * WN * 64, (BM / WM / 16) * (BN / WN / 16) <= 16
   const int64_t m0 = (tile / tiles_n) * BM, n0 = (tile % tiles_n) * BN;
 
   if (!wgrad_schedule<Cfg::NT>(p, slot_id, sched, reinterpret_cast<int32_t*>(ring),
-                               p.order == kWgOrderChunkXcd))
+                               p.order == kWgOrderChunkXcd ? kWgSortRoutes16 : kWgNoSort))
     return;
   const int32_t expert = __builtin_amdgcn_readfirstlane(sched.expert);
   const int64_t lo = sched.lo, hi = sched.hi;

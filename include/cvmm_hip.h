@@ -97,13 +97,17 @@ int cvmm_timing_result(uint32_t kernel_class, double* total_ms, int64_t* launche
  *     1 = the tiles of one expert chunk on one XCD, 2 = one dW tile of every
  *     expert on one XCD, 3 = expert chunk c on XCD c % 8 with all its tiles.
  *     Built in: 3 for the 16-bit kernel's 128 x 128 and 256 x 256 dW tiles
- *     (3 starts the longest chunks first, in up to 256 experts), else 2.
+ *     (3 starts the longest chunks first, in 9 to 256 experts of 768 or more
+ *     routes each on average), else 2.  The fp32 kernel starts the longest
+ *     chunks first in both of its orders: 3, built in from 64 experts, and 1,
+ *     a chunk's tiles over all XCDs (2 is the same there).
  *   CVMM_TUNE_WGRAD_TILE: dW tile of the 16-bit weight-gradient kernel where
  *     its base tile is 128 x 128 and dW is contiguous aligned fp32: 1 = 128 x
  *     128, 2 = 256 x 128, 3 = 128 x 256, 4 = 256 x 256 of four waves, 5 =
  *     256 x 256 of eight waves.  Built in: 256 x 256 of eight waves when
  *     d_in, d_out >= 256 and the experts' tiles fill about four rounds of
- *     256 CUs, or two with >= 512 routes per expert.
+ *     256 CUs, or two with >= 512 routes per expert where those tiles cover
+ *     at most 1.15 times the area of the 128 x 128 ones.
  *   CVMM_TUNE_GEMM_ORDER: m-tile order of the routed GEMMs (forward, grad
  *     input), 1 = expert-major, 2 = token-major (tile j of every expert next
  *     to each other; up to 256 experts).  Built in: token-major for the

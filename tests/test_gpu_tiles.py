@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import cvmm_codex_amd.api as C
+from cvmm_codex_amd import _native as N
 from tests import gpu_util as U
 
 pytestmark = pytest.mark.gpu
@@ -46,8 +47,7 @@ def test_surplus_tiles_zero_the_unrouted_rows(E):
 @pytest.mark.parametrize("E", [1, 5, 16])
 @pytest.mark.parametrize("load", ["even", "one_long", "one_empty"])
 def test_weight_gradient_chunk_order(E, load):
-    # 400 routes per expert: chunks run longest first if some expert has more
-    # than 1.25 times the mean, else in expert order
+    # 400 routes per expert: below the loads whose chunks are ordered by length
     g = torch.Generator().manual_seed(E)
     T, K, D, H = 100 * E, 4, 136, 128
     sel = (torch.arange(T * K) % E).view(T, K)
@@ -61,3 +61,49 @@ def test_weight_gradient_chunk_order(E, load):
     got = U.run_hip(x, keys, sel, None, go, False, True)
     exp = U.run_oracle(x, keys, sel, None, go, False, True)
     U.compare(got, exp, 2e-2)
+
+
+def _dw64(x, ids, go, E):
+    """dW[e] = sum over the routes of e of x^T go in float64."""
+    order = torch.argsort(ids.reshape(-1), stable=True)
+    rows = x.double()[order // ids.shape[1]].split(torch.bincount(ids.reshape(-1), minlength=E).tolist())
+    g = go.double().reshape(-1, go.shape[-1])[order].split([r.shape[0] for r in rows])
+    return torch.stack([a.T @ b for a, b in zip(rows, g)])
+
+
+@pytest.mark.parametrize("E", [8, 9, 16, 64, 65, 128, 200, 256, 257])
+@pytest.mark.parametrize("load,chunk", [("even", 0), ("uneven", 0), ("uneven", 256), ("one_long", 512)])
+def test_weight_gradient_chunks_by_length(E, load, chunk):
+    """800 routes per expert: with 9 to 256 experts of uneven loads the chunks
+    run longest first (the rank spans one to four waves), split experts among
+    them; other launches in expert order.  The bits of the tile-major order,
+    which never sorts, and float64's sums within fp32's rounding of ~800
+    terms."""
+    g = torch.Generator().manual_seed(E)
+    K, D, H = 4, 72, 136
+    T = 200 * E
+    ids = (torch.arange(T * K) % E).view(T, K)
+    if load == "uneven":
+        ids = torch.multinomial(1 + 1.5 * torch.rand(E, generator=g), T * K, replacement=True, generator=g).view(T, K)
+        ids[ids == 1] = 0          # an empty expert
+    elif load == "one_long":
+        ids[torch.rand(T, K, generator=g) < 0.3] = E // 2
+    x = torch.randn(T, D, generator=g).to(torch.bfloat16).cuda()
+    keys = torch.randn(E, D, H, generator=g).cuda().requires_grad_()
+    go = torch.randn(T, K, H, generator=g).to(torch.bfloat16).cuda()
+    ids = ids.cuda()
+    lib = N.lib()
+    out = []
+    assert lib.cvmm_tuning_set(N.TUNE_WGRAD_CHUNK, chunk) == 0
+    try:
+        for order in (0, 2):
+            assert lib.cvmm_tuning_set(N.TUNE_WGRAD_ORDER, order) == 0
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                y = C.cvmm(x, C.cvmm_prepare_sel2(ids), keys)
+            out.append(torch.autograd.grad(y, keys, go)[0])
+    finally:
+        lib.cvmm_tuning_set(N.TUNE_WGRAD_ORDER, 0)
+        lib.cvmm_tuning_set(N.TUNE_WGRAD_CHUNK, 0)
+    assert torch.equal(out[0], out[1])
+    ref = _dw64(x, ids, go, E)
+    assert ((out[0].double() - ref).abs().max() / ref.abs().max()).item() <= 1e-5
