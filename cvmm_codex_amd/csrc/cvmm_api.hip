@@ -90,13 +90,21 @@ static std::atomic<int64_t> g_wgrad_chunk{0};
 void wgrad_geometry(int64_t M, int64_t N, int64_t n_routes, int32_t n_experts, int32_t op_dtype, int64_t* split,
                     int64_t* grid_chunks, int64_t* max_slots, int64_t* tiles_mn) {
   const int64_t bk = op_dtype == kF32 ? 32 : 64;
-  // chunk = max(1024, one CU's share of the launch: R x tiles / 256 CUs).  A
-  // longer expert alone would outlast the rest of the launch; a shorter chunk
-  // adds an fp32 partial of the expert's dW, written and read back.  Measured
-  // (longest chunk first, cvmm_wgrad_sched.h): ff_up with loads up to 2.2x
-  // the mean, share 2048: 46 us against 51 / 67 / 73 at 1536 / 1280 / 1024
-  // and 57 at 3072; the FFN stack (Zipf loads up to 16x), share 8192: 434 us
-  // per launch against 521 / 462 / 558 at 6144 / 12288 / 16384.
+  // chunk = one CU's share of the launch, R x tiles / 256 CUs, at least 1024
+  // routes (256 in fp32, whose MFMAs take 16 times as long).  A longer expert
+  // alone would outlast the rest of the launch; a shorter chunk adds an fp32
+  // partial of the expert's dW, written and read back.  Measured (longest
+  // chunk first, cvmm_wgrad_sched.h): ff_up with loads up to 2.2x the mean,
+  // share 2048: 46 us against 51 / 67 / 73 at 1536 / 1280 / 1024 and 57 at
+  // 3072; the FFN stack (Zipf loads up to 16x), share 8192: 434 us per launch
+  // against 521 / 462 / 558 at 6144 / 12288 / 16384.  fp32, 512 x 256, 4096
+  // routes on 4 experts, share 256: 25 us, 55 in chunks of 1024.
+  // Where that share is about the mean load, half the experts would be split
+  // to save less than the ~10 us that a split costs (450 routes of a 128 x
+  // 128 tile, 200 of an fp32 one): there an expert stays whole up to 1.5 times
+  // the mean (1.1 in fp32).  32 experts of 1024 x 128, 32768 routes drawn
+  // evenly: 39 us split at the share, 29 whole; fp32, 16 of them, 16384
+  // routes: 87 and 63 (73 and 77 with loads up to 1.4 times the mean).
   int bm, bn;
   if (op_dtype == kF32) f32_wgrad_tile(M, N, n_experts, &bm, &bn);
   else wgrad_fast_tile(M, N, wgrad_auto_tile(M, N, n_routes, n_experts), &bm, &bn);
@@ -104,8 +112,13 @@ void wgrad_geometry(int64_t M, int64_t N, int64_t n_routes, int32_t n_experts, i
   const int64_t knob = g_wgrad_chunk.load();
   int64_t s = knob;
   if (s <= 0) {
-    s = (int64_t)((double)n_routes * (double)tiles / 256.0);
-    if (s < 1024) s = 1024;
+    const bool f32 = op_dtype == kF32;
+    const double share = (double)n_routes * (double)tiles / 256.0;
+    const double mean = n_experts > 0 ? (double)n_routes / n_experts : 0.0;
+    const double whole = (f32 ? 1.1 : 1.5) * mean;
+    s = (int64_t)share;
+    if (1.1 * mean - share < (f32 ? 200.0 : 450.0) && s < (int64_t)whole) s = (int64_t)whole;
+    if (s < (f32 ? 256 : 1024)) s = f32 ? 256 : 1024;
     if (s > n_routes && n_routes > 0) s = n_routes;
   }
   s = (s + bk - 1) / bk * bk;
