@@ -829,9 +829,13 @@ int cvmm_sort_routes_cast_keys_ex(const void* sel, int32_t sel_is_int64, int64_t
 }  // extern "C"
 
 // (an output of another type than the op's, or summed by atomics, stays with
-// the general kernels)
+// the general kernels; so does an unweighted short-K product below 3e8, which
+// the two copies' launches outweigh: 4096 routes, 8 / 64 experts, 100 -> 500
+// 36 / 35 us per call, 40 / 40 padded; 100 -> 1001 40 / 62 and 40 / 44.  A
+// weighted one pays the combine's launch either way: 47 and 44)
 static bool fwd_pads(int32_t op_dtype, int32_t out_dtype, int64_t n_routes, int32_t n_experts, int64_t d_in,
-                     int64_t d_out, int32_t flags) {
+                     int64_t d_out, bool weighted, int32_t flags) {
+  if (!weighted && d_in <= 128 && (double)n_routes * (double)d_in * (double)d_out < 3.0e8) return false;
   return out_dtype == op_dtype && !(flags & CVMM_FLAG_ATOMIC_REDUCE) &&
          pads_operands(op_dtype, n_routes, n_experts, d_in, d_out);
 }
@@ -847,7 +851,7 @@ size_t cvmm_fwd_workspace_bytes(int64_t n_routes, int32_t n_experts, int64_t d_i
                      use_dense_topk(op_dtype, out_rows, n_experts, d_in, d_out, k);
   if (dense) carve_dense(c, out_rows, n_experts, d_in, d_out, n_routes, op_dtype);
   if (!has_offsets) c.take((size_t)n_experts * 8);
-  const bool padded = fwd_pads(op_dtype, out_dtype, n_routes, n_experts, d_in, d_out, flags);
+  const bool padded = fwd_pads(op_dtype, out_dtype, n_routes, n_experts, d_in, d_out, weighted, flags);
   if (weighted && !dense) {
     if (flags & CVMM_FLAG_ATOMIC_REDUCE) {
       c.take((size_t)out_rows * d_out * 4);
@@ -933,7 +937,7 @@ static int fwd_core(const void* x, int32_t x_dtype, int64_t x_rows, int64_t x_ld
   p.token_major = gemm_token_major(n_experts);
 
   // the route buffer of a weighted call comes before the padded copies
-  const bool pad_sizes = !dense && fwd_pads(op_dtype, out_dtype, n_routes, n_experts, d_in, d_out, flags);
+  const bool pad_sizes = !dense && fwd_pads(op_dtype, out_dtype, n_routes, n_experts, d_in, d_out, weighted, flags);
   const int64_t out_w = pad_sizes ? pad8(d_out) : d_out;
   void* ybuf = nullptr;
   int32_t* inv_ws = nullptr;

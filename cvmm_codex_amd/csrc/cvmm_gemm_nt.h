@@ -407,11 +407,16 @@ hipError_t launch_routed_gemm_nt_op(const GemmParams& p, hipStream_t stream) {
   // one k stage per tile (K <= 64): walk all n-tiles of an m-tile in one
   // workgroup (plain stores only).  Measured: switch_o forward 2.07 -> 1.51 ms;
   // with two k stages (K = 128, ff_up grad-input) the tiled kernel is faster.
+  // Where the m-tiles fill less than two workgroups per CU, several share an
+  // m-tile's n-tiles (4096 routes over 8 experts, 64 -> 2008: 110 -> 26 us).
   const int64_t nk = (p.K + 63) / 64;
   const int64_t n_ntiles = (p.N + 127) / 128;
   if (nk == 1 && n_ntiles > 1 && p.epi == kEpiStore && p.dg == nullptr && p.out != nullptr && p.N % 8 == 0 &&
-      p.n_out == p.N && p.out_ld % 8 == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0)
-    return launch_routed_gemm_nloop_t<OpT, 128, 128>(p, (int32_t)n_ntiles, stream);
+      p.n_out == p.N && p.out_ld % 8 == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0) {
+    int64_t groups = p.grid_tiles > 0 ? (2 * 256 + p.grid_tiles - 1) / p.grid_tiles : 1;
+    if (groups > n_ntiles) groups = n_ntiles;
+    return launch_routed_gemm_nloop_t<OpT, 128, 128>(p, (int32_t)((n_ntiles + groups - 1) / groups), stream);
+  }
   return launch_routed_gemm_nt_t<OpT, 128, 128>(p, stream);
 }
 

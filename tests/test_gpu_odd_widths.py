@@ -43,6 +43,8 @@ def _run(T, K, D, H, E, weighted, route_input, xdt, kdt, op, hot):
     (1400, 8, 60, 1024),    # that can keep scaled route rows: here p.K != d_in, none are kept)
     (1400, 8, 126, 1020),
     (1400, 8, 64, 1020),    # the same with only d_out off the grid
+    (1024, 4, 33, 1001),    # a K <= 64 product over groups of column tiles (weighted)
+    (700, 8, 100, 250),     # an unweighted forward that stays with the general kernel
 ])
 @pytest.mark.parametrize("weighted,route_input", [(False, False), (True, True), (True, False), (False, True)])
 def test_padded_widths(T, K, D, H, weighted, route_input):

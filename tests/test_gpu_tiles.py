@@ -107,3 +107,19 @@ def test_weight_gradient_chunks_by_length(E, load, chunk):
     assert torch.equal(out[0], out[1])
     ref = _dw64(x, ids, go, E)
     assert ((out[0].double() - ref).abs().max() / ref.abs().max()).item() <= 1e-5
+
+
+@pytest.mark.parametrize("T,k,E,D,H", [(64, 2, 8, 64, 1000), (300, 2, 8, 40, 136), (1024, 4, 8, 64, 2008),
+                                       (40, 1, 70, 24, 520)])
+def test_short_products_over_groups_of_column_tiles(T, k, E, D, H):
+    """K <= 64 and N off the 64-column grid: the workgroups of a launch with
+    few row tiles share out its column tiles."""
+    g = torch.Generator().manual_seed(T + H)
+    x = torch.randn(T, k, D, generator=g).to(torch.bfloat16)
+    keys = torch.randn(E, D, H, generator=g) / D ** 0.5
+    ids = torch.randint(0, E, (T, k), generator=g)
+    w = torch.rand(T, k, generator=g)
+    go = torch.randn(T, H, generator=g).to(torch.bfloat16)
+    got = U.run_hip(x, keys, ids, w, go, True, True)
+    exp = U.run_oracle(x, keys, ids, w, go, True, True)
+    U.compare(got, exp, 2e-2)
