@@ -101,12 +101,14 @@ struct RouteSortOut {
   int32_t* route_pos;    // or NULL
 };
 
-// Routes of one router workgroup, at most: a chunk of >= 512 routes in whole
-// tokens of up to kRouteMaxK (route_chunk_tokens).
-constexpr int kRouteOneMax = 512 + (int)kRouteMaxK;
+// Routes that a single router workgroup sorts itself, at most.  Beyond them
+// its ranking outlasts a second launch: 64 tokens, top-8, 128 / 256 / 512
+// experts 26 / 42 / 76 us per call in one launch, 23 / 38 / 73 in two; 32
+// tokens 14 / 22 / 39 and 20 / 23 / 41.
+constexpr int kRouteOneMax = 256;
 static_assert(kRouteOneMax % 64 == 0, "whole waves of ids");
 
-// ONE: a single workgroup routes every token (a decode step: up to 512
+// ONE: a single workgroup routes every token (a decode step: up to 256
 // routes) and sorts the routes itself -- the histogram's scan in LDS, then
 // each route's rank among the earlier routes of its expert, counted over the
 // ids in LDS -- instead of leaving the counts to a second launch.  At 4 and 32

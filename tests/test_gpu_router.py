@@ -204,11 +204,13 @@ def test_gate_logits_against_the_torch_projection(T, D, E, amp):
 
 
 @pytest.mark.parametrize("T,E,k", [(1, 1, 1), (1, 64, 8), (4, 128, 8), (64, 128, 8), (8, 1024, 64), (9, 100, 64),
-                                   (512, 3, 1), (513, 3, 1), (170, 33, 3), (171, 33, 3), (65, 128, 8)])
+                                   (512, 3, 1), (513, 3, 1), (170, 33, 3), (171, 33, 3), (65, 128, 8),
+                                   (32, 128, 8), (33, 128, 8), (256, 3, 1), (257, 3, 1), (85, 33, 3), (86, 33, 3),
+                                   (4, 1024, 64), (5, 1024, 64)])
 def test_router_sort_around_one_workgroup(T, E, k):
-    """The router that sorts its own routes (up to one chunk of 512 routes in
-    whole tokens) and the two-launch form past it: the selector equals the
-    stable sort of the returned ids."""
+    """The router that sorts its own routes (up to 256) and the two-launch form
+    past it, of one chunk and of two: the selector equals the stable sort of
+    the returned ids."""
     g = torch.Generator().manual_seed(T + E + k)
     logits = torch.randn(T, E, generator=g)
     logits[T // 2] = 1.0   # ties: lower ids first
