@@ -28,6 +28,7 @@ host sync).
 """
 from __future__ import annotations
 
+import functools
 import os
 import threading
 from dataclasses import dataclass
@@ -152,15 +153,18 @@ class _CopyPlan(NamedTuple):
     layout: int  # N.CAST_*_INTERLEAVED bits
     fwd_t: bool
     bwd_t: bool
-    stored: bool = False
+    stored: bool
+    cast_n: bool  # kn is a copy
+    casts: bool   # there is a copy to cast
 
-    @property
-    def cast_n(self) -> bool:
-        return self.want_n and not self.stored
 
-    @property
-    def casts(self) -> bool:
-        return self.want_t or self.cast_n
+def _new_plan(want_t: bool, want_n: bool, layout: int, fwd_t: bool, bwd_t: bool, stored: bool = False) -> _CopyPlan:
+    cast_n = want_n and not stored
+    return _CopyPlan(want_t, want_n, layout, fwd_t, bwd_t, stored, cast_n, want_t or cast_n)
+
+
+# an eager call takes its plan from the few dozen there are
+_kept_plan = functools.lru_cache(None)(_new_plan)
 
 
 def _sort_routes_cast(raw_flat: torch.Tensor, n_experts: int, top_k: int, cast, counted_ws=None):
@@ -199,13 +203,6 @@ def _copies(keys: torch.Tensor, op: torch.dtype, plan: _CopyPlan):
     return kt, (keys.detach() if plan.stored else kn)
 
 
-def _rows_in_place(keys: torch.Tensor) -> bool:
-    """The keys' rows of d_out values can be read 16 bytes at a time."""
-    per = 16 // keys.element_size()
-    return (keys.stride(2) == 1 and keys.stride(1) % per == 0 and keys.stride(0) % per == 0
-            and keys.data_ptr() % 16 == 0)
-
-
 @torch._dynamo.assume_constant_result
 def _topk_dense(n_tokens: int, n_experts: int, K: int, N_: int, top_k: int, op_id: int) -> bool:
     """Whether the library takes this top-k sum as one dense GEMM
@@ -224,13 +221,13 @@ def _plan_copies(keys: torch.Tensor, op: torch.dtype, n_routes: int, top_k: int,
                  and _topk_dense(T, E, d_out, d_in, top_k, op_id))
     if _compiling():
         fwd_t, bwd_t = not fwd_dense, bwd_dense
-        return _CopyPlan(fwd_t or (need_grad_input and bwd_t), (not fwd_t) or (need_grad_input and not bwd_t),
+        return _new_plan(fwd_t or (need_grad_input and bwd_t), (not fwd_t) or (need_grad_input and not bwd_t),
                          0, fwd_t, bwd_t)
-    return _eager_plan(keys, op, n_routes, fwd_dense, bwd_dense, need_grad_input)
+    return _eager_plan(keys, op, n_routes, fwd_dense, bwd_dense, need_grad_input, weighted and cvmm_atomic_reduce)
 
 
 def _eager_plan(keys: torch.Tensor, op: torch.dtype, n_routes: int, fwd_dense: bool, bwd_dense: bool,
-                need_grad_input: bool) -> _CopyPlan:
+                need_grad_input: bool, atomic: bool = False) -> _CopyPlan:
     """Eager copies: one copy where one product runs the long-K routed GEMM
     (K > 128), which reads the weights in either orientation, and the other
     product needs that copy's own orientation (the short-K kernel's, or a
@@ -239,23 +236,25 @@ def _eager_plan(keys: torch.Tensor, op: torch.dtype, n_routes: int, fwd_dense: b
     a forward alone reads the weights as they are stored wherever a kernel
     takes them so (cvmm_fwd_stored_keys): casting every expert's weights took
     two thirds of a 32-token decode step (447 of 686 us over 128 experts of
-    2048 x 512 in bf16) and of a 1999-token prefill (449 of 768 us)."""
-    E, d_in, d_out = keys.shape
-    in_place = keys.dtype == op and _rows_in_place(keys)
+    2048 x 512 in bf16) and of a 1999-token prefill (449 of 768 us).  `atomic`:
+    the top-k sum is made by fp32 atomics, whose kernel reads in-place weights
+    more slowly than a copy: 4 tokens, 64 experts of 1024 x 128 in bf16 48 us
+    with the copy, 53 without, 128 experts of 2048 x 512 281 and 138."""
     layout = (N.CAST_T_INTERLEAVED if fwd_dense else 0) | (N.CAST_N_INTERLEAVED if bwd_dense else 0)
     if not need_grad_input:
-        if (not fwd_dense and (in_place or (keys.dtype == torch.float32 and _rows_in_place(keys)))
-                and N.lib().cvmm_fwd_stored_keys(n_routes, E, d_in, d_out, _DTYPE_IDS[keys.dtype], _DTYPE_IDS[op])):
-            return _CopyPlan(False, True, 0, False, False, True)
-        return _CopyPlan(True, False, layout, True, False)
+        if (not fwd_dense and not (atomic and keys.numel() < 1 << 25)
+                and N.host().keys_in_place(keys, n_routes, _DTYPE_IDS[op]) & 2):
+            return _kept_plan(False, True, 0, False, False, True)
+        return _kept_plan(True, False, layout, True, False)
+    _, d_in, d_out = keys.shape
     fwd_ring = d_in > 128 and not fwd_dense
     bwd_ring = d_out > 128 and not bwd_dense
-    stored = in_place and not bwd_dense
+    stored = not bwd_dense and keys.dtype == op and bool(N.host().keys_in_place(keys, n_routes, _DTYPE_IDS[op]) & 1)
     if fwd_ring:       # kn only: the forward reads it n-contiguous
-        return _CopyPlan(False, True, layout, False, False, stored)
+        return _kept_plan(False, True, layout, False, False, stored)
     if bwd_ring:       # kt only: the grad-input reads it n-contiguous
-        return _CopyPlan(True, False, layout, True, True)
-    return _CopyPlan(True, True, layout, True, False, stored)
+        return _kept_plan(True, False, layout, True, True)
+    return _kept_plan(True, True, layout, True, False, stored)
 
 
 def _copy_view(plan: _CopyPlan, kt, kn, fwd: bool):
@@ -958,7 +957,7 @@ def _cvmm_eager(x: torch.Tensor, sel: Union[torch.Tensor, CVMMSel], keys: torch.
         fwd_dense = weighted and k >= 2 and not cvmm_atomic_reduce and _topk_dense(T, E, d_in, d_out, k, op_id)
         bwd_dense = (need and not weighted and token_input and k >= 2 and not cvmm_atomic_reduce
                      and _topk_dense(T, E, d_out, d_in, k, op_id))
-        plan = _eager_plan(keys, op, raw.numel(), fwd_dense, bwd_dense, need)
+        plan = _eager_plan(keys, op, raw.numel(), fwd_dense, bwd_dense, need, weighted and cvmm_atomic_reduce)
     if pending:
         sel._resolve(E, (keys, op, plan) if plan is not None and plan.casts else None)
     _log_shape(x, keys)

@@ -311,6 +311,22 @@ Tensor expert_offsets(const Tensor& sorted, int64_t n_experts, int64_t stream) {
   return out;
 }
 
+// Which uses read the keys as they are stored (see _eager_plan in api.py).
+// Bit 0: in place of the [E, d_in, d_out] copy (keys of the op dtype, rows of
+// d_out values that 16-byte pieces can be read from); bit 1: in a forward of
+// n_routes alone (cvmm_fwd_stored_keys, for fp32 or op-dtype keys).
+int64_t keys_in_place(const Tensor& keys, int64_t n_routes, int64_t op_id) {
+  const auto op = dtype_of(op_id), kd = keys.scalar_type();
+  const int64_t per = 16 / keys.element_size();
+  if ((kd != op && kd != at::kFloat) || keys.stride(2) != 1 || keys.stride(1) % per != 0 ||
+      keys.stride(0) % per != 0 || (reinterpret_cast<uintptr_t>(keys.data_ptr()) & 15) != 0)
+    return 0;
+  return (kd == op ? 1 : 0) | (cvmm_fwd_stored_keys(n_routes, (int32_t)keys.size(0), keys.size(1), keys.size(2),
+                                                    dtype_id(kd), (int32_t)op_id) != 0
+                                   ? 2
+                                   : 0);
+}
+
 // keys [E, d_in, d_out] -> op-dtype copies kt (forward) and kn (grad-input)
 // in the layouts of cast_outputs, one pass.
 std::tuple<OptT, OptT> cast_keys(const Tensor& keys, int64_t op_id, bool want_t, bool want_n, int64_t layout,
@@ -796,6 +812,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sort_routes_cast", &sort_routes_cast, py::arg("raw"), py::arg("n_experts"), py::arg("top_k"),
         py::arg("keys"), py::arg("op_id"), py::arg("want_t"), py::arg("want_n"), py::arg("layout"),
         py::arg("stream"), py::arg("counted_ws") = py::none());
+  m.def("keys_in_place", &keys_in_place);
   m.def("cast_keys", &cast_keys, py::arg("keys"), py::arg("op_id"), py::arg("want_t"), py::arg("want_n"),
         py::arg("layout"), py::arg("stream"));
   m.def("forward", &forward_py);

@@ -162,3 +162,51 @@ def test_gate_logits_has_no_cpu_path():
     """cvmm_gate_logits, like the products, takes device tensors only."""
     with pytest.raises(RuntimeError, match="no CPU fallback"):
         C.cvmm_gate_logits(torch.randn(4, 8), torch.randn(8, 3))
+
+
+def test_keys_in_place_over_layouts():
+    """Which weights are read as they are stored: rows of unit stride that
+    start at multiples of 16 bytes, of the op dtype (bit 0) or, in a forward of
+    few routes, fp32 too (bit 1)."""
+    from cvmm_codex_amd import _native as N
+    f = N.host().keys_in_place
+    E, D, H = 4, 136, 72
+    bf, f32 = N.dtype_id(torch.bfloat16), N.dtype_id(torch.float32)
+
+    def flat(dtype, extra):
+        t = torch.zeros(E * D * H + 64, dtype=dtype)
+        pad = (-t.data_ptr() // t.element_size()) % (16 // t.element_size())
+        return t[pad + extra:pad + extra + E * D * H].view(E, D, H)
+
+    k16, k32 = flat(torch.bfloat16, 0), flat(torch.float32, 0)
+    assert f(k16, 8, bf) == 3 and f(k16, 10 ** 6, bf) == 3          # d_in > 128: the long-K kernel takes them
+    assert f(k16[:, :64], 8, bf) == 3 and f(k16[:, :64], 10 ** 6, bf) == 1
+    assert f(k32, 8, bf) == 2 and f(k32, 10 ** 6, bf) == 0
+    assert f(k32, 8, f32) == 1                                      # no fp32 kernel streams them
+    assert f(k16, 8, N.dtype_id(torch.float16)) == 0                # another 16-bit type
+    assert f(flat(torch.bfloat16, 1), 8, bf) == 0 and f(flat(torch.float32, 2), 8, bf) == 0
+    assert f(flat(torch.bfloat16, 8), 8, bf) == 3
+    assert f(k16.transpose(1, 2), 8, bf) == 0
+    assert f(torch.stack([k16, k16], -1)[..., 0], 8, bf) == 0
+    assert f(k16[..., 8:], 8, bf) == 3 and f(k16[..., 4:], 8, bf) == 0
+    assert f(k16[:1].expand(E, D, H), 8, bf) == 3                   # one matrix for every expert
+    assert f(k16.double(), 8, bf) == 0
+
+
+@pytest.mark.parametrize("need", [False, True])
+@pytest.mark.parametrize("fwd_dense,bwd_dense", [(False, False), (True, False), (False, True)])
+def test_stored_plans_read_only_what_is_there(need, fwd_dense, bwd_dense):
+    """Every plan over layouts and sizes has the copy (or the keys) that each
+    phase reads."""
+    for dtype in (torch.float32, torch.bfloat16):
+        for d_in, d_out in ((64, 64), (64, 256), (256, 64), (256, 256)):
+            for n_routes in (4, 10 ** 5):
+                for atomic in (False, True):
+                    keys = torch.zeros(4, d_in, d_out, dtype=dtype)
+                    p = C._eager_plan(keys, torch.bfloat16, n_routes, fwd_dense, bwd_dense, need, atomic)
+                    assert p.want_t if p.fwd_t else p.want_n
+                    if need:
+                        assert p.want_t if p.bwd_t else p.want_n
+                    assert not (p.stored and atomic and not need)
+                    assert not (p.stored and dtype == torch.float32 and (need or n_routes > 1000))
+                    assert p.casts == (p.want_t or (p.want_n and not p.stored))

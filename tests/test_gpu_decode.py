@@ -116,3 +116,21 @@ def test_no_scaled_rows_are_made_where_none_are_kept(T, k, E, D, H, weights):
 
     training, frozen = made(keys.clone().requires_grad_()), made(keys)
     assert training == frozen
+
+
+@pytest.mark.parametrize("weights", ["fp32", "bf16"])
+@pytest.mark.parametrize("E,D,H", [(8, 136, 128), (64, 1024, 512)])   # weights below and from 2^25 values
+def test_atomic_sums_over_stored_weights(monkeypatch, E, D, H, weights):
+    """The top-k sum by atomics copies small weights and reads large ones in place."""
+    monkeypatch.setattr(C, "cvmm_atomic_reduce", True)
+    T, k = 9, 3
+    _, keys, sel = _case(T, k, E, D, H, "bf16", weights, False, E)
+    x = torch.randn(T, k, D, device="cuda").to(torch.bfloat16)
+    w = torch.rand(T, k, device="cuda")
+    plan = C._eager_plan(keys, torch.bfloat16, T * k, False, False, False, True)
+    assert plan.stored == (keys.numel() >= 1 << 25)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        y = C.cvmm(x, C.cvmm_prepare_sel2(sel, w, route_input=True), keys)
+    kd = keys.to(torch.bfloat16).double()
+    ref = torch.stack([sum(w[t, j].double() * (x[t, j].double() @ kd[sel[t, j]]) for j in range(k)) for t in range(T)])
+    _check(y, ref)
