@@ -95,16 +95,25 @@ __device__ bool gemm_schedule_tile(const GemmParams& p, int64_t n_groups, RouteM
     if (p.n_experts <= kTokenMajorMaxExperts) {
       int64_t st[G], en[G];
       int32_t nt[G], incl[G], ntmax = 0;
+      // (groups of 64 past the last expert are skipped: the four groups'
+      // clamps and scans in every workgroup cost a 64-expert launch ~1 us)
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        range(g * 64 + lane, st[g], en[g]);
-        nt[g] = tiles_of(st[g], en[g]);
-        ntmax = nt[g] > ntmax ? nt[g] : ntmax;
+        st[g] = en[g] = 0;
+        nt[g] = 0;
+        if (g * 64 < p.n_experts) {
+          range(g * 64 + lane, st[g], en[g]);
+          nt[g] = tiles_of(st[g], en[g]);
+          ntmax = nt[g] > ntmax ? nt[g] : ntmax;
+        }
       }
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        incl[g] = wave_incl_scan(nt[g]) + n_tiles;
-        n_tiles = __builtin_amdgcn_readlane(incl[g], 63);
+        incl[g] = n_tiles;
+        if (g * 64 < p.n_experts) {
+          incl[g] += wave_incl_scan(nt[g]);
+          n_tiles = __builtin_amdgcn_readlane(incl[g], 63);
+        }
       }
       locate();
       if (tile < n_tiles && p.token_major > 0) {
