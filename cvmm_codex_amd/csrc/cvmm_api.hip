@@ -135,6 +135,10 @@ int32_t wgrad_auto_tile(int64_t M, int64_t N, int64_t n_routes, int32_t n_expert
   if (M < 256 || N < 256) return kWgTileBase;
   const int64_t m = (M + 255) / 256, n = (N + 255) / 256;
   const int64_t wide = n_experts * m * n;
+  // about four rounds of CUs.  Evenly loaded experts of 2048 x 512 that draw
+  // 300 routes each, 128-wide / wide: 55 experts (880 wide tiles) 100 / 92 us,
+  // 64 127 / 107.  (Fewer gain too, 46 experts 84 / 74, 40 73 / 70; 24, of 700
+  // routes each, do not, 79 / 81.  The line is not drawn there yet.)
   if (7 * wide >= 6 * 4 * 256) return kWgTile256x256W8;
   // two rounds of CUs where the experts are long and the wide tiles cover
   // little more than the base ones (8 experts of 1024 x 4096, 1024 routes
