@@ -105,6 +105,14 @@ void wgrad_geometry(int64_t M, int64_t N, int64_t n_routes, int32_t n_experts, i
   // the mean (1.1 in fp32).  32 experts of 1024 x 128, 32768 routes drawn
   // evenly: 39 us split at the share, 29 whole; fp32, 16 of them, 16384
   // routes: 87 and 63 (73 and 77 with loads up to 1.4 times the mean).
+  // Short launches split less readily too: their last workgroups wait for the
+  // partials.  256 x 256 tiles up to 800 routes past the share (64 experts of
+  // 2048 x 512, share 1250, the longest expert 1388 / 1757 routes: 122 / 129 us
+  // split at the share, 116 / 125 whole; 32, share 2048, 2648: 128 and 115;
+  // from 4096 on, or with few experts, whose chunks even out the XCDs, the
+  // share itself), others up to 1408 where the share is shorter than 1024 and
+  // no CU idles (20 experts of 512 x 1024, 8000 routes, the longest 1075 / 1273
+  // / 1729: 39 / 39 / 41 split at 1024, 33 / 36 / 42 whole).
   int bm, bn;
   if (op_dtype == kF32) f32_wgrad_tile(M, N, n_experts, &bm, &bn);
   else wgrad_fast_tile(M, N, wgrad_auto_tile(M, N, n_routes, n_experts), &bm, &bn);
@@ -117,6 +125,8 @@ void wgrad_geometry(int64_t M, int64_t N, int64_t n_routes, int32_t n_experts, i
     const double mean = n_experts > 0 ? (double)n_routes / n_experts : 0.0;
     const double whole = (f32 ? 1.1 : 1.5) * mean;
     s = (int64_t)share;
+    if (!f32 && bm == 256 && bn == 256 && n_experts >= 16 && share < 4096.0) s += 800;
+    if (!f32 && share < 1024.0 && share >= mean && s < 1408) s = 1408;
     if (1.1 * mean - share < (f32 ? 200.0 : 450.0) && s < (int64_t)whole) s = (int64_t)whole;
     if (s < (f32 ? 256 : 1024)) s = f32 ? 256 : 1024;
     if (s > n_routes && n_routes > 0) s = n_routes;

@@ -129,6 +129,7 @@ int cvmm_timing_result(uint32_t kernel_class, double* total_ms, int64_t* launche
  *     summed in chunk order).  Built in: one CU's share of the launch,
  *     routes x dW tiles / 256, at least 1024 (fp32: 256), and 1.5 (fp32: 1.1)
  *     times the mean routes per expert where the share is about that mean.
+ *     Short launches of 16-bit types take somewhat longer chunks.
  *     Workspace queries depend on it: query after setting it.
  *   CVMM_TUNE_RING_TILE: tile of the long-K routed GEMM (K > 128, N > 64):
  *     1 = 128 x 128, 2 = 160 x 128, 3 = 256 x 256 of eight waves where N is

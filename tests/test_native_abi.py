@@ -90,6 +90,37 @@ def test_row_copy_queries(lib):
     assert lib.cvmm_bwd_w_workspace_bytes_ex(32760, 63, 412, 130, N.BF16, 1, 0) >= base + need
 
 
+@pytest.mark.parametrize("op,R,E,D,H,chunk", [
+    (N.BF16, 65536, 64, 1024, 128, 2048),      # one CU's share: R x 8 tiles / 256
+    (N.BF16, 32768, 32, 1024, 128, 1536),      # the share is the mean: 1.5 times it
+    (N.BF16, 32768, 8, 512, 512, 2048),        # half the mean: CUs would idle
+    (N.BF16, 4096, 4, 1024, 128, 1024),        # a short share of idle CUs
+    (N.BF16, 8000, 20, 512, 1024, 1408),       # a short share of busy ones
+    (N.BF16, 20000, 64, 2048, 512, 2112),      # 256 x 256 tiles: 800 past the share
+    (N.BF16, 131072, 128, 2048, 512, 8192),    # ... not from a share of 4096 on
+    (N.BF16, 8192, 8, 1024, 4096, 2048),       # ... nor for few experts
+    (N.F32, 32768, 64, 1024, 128, 2048),
+    (N.F32, 4096, 4, 512, 256, 256),
+    (N.F32, 16384, 16, 1024, 128, 1152),       # the share is the mean: 1.1 times it
+])
+def test_weight_gradient_chunk_rule(lib, op, R, E, D, H, chunk):
+    """The built-in chunk length on both sides of each line of its rule, read
+    from the partial slots (2 R / chunk + 1) the workspace holds."""
+    def size(knob):
+        assert lib.cvmm_tuning_set(N.TUNE_WGRAD_CHUNK, knob) == 0
+        return lib.cvmm_bwd_w_workspace_bytes(R, E, D, H, op, 1)
+
+    try:
+        unit = size(R // 2 // 64 * 64) - size(2 * R)     # 5 slots (or 4), 2
+        slots_half = 2 * R // (R // 2 // 64 * 64) + 1
+        unit //= slots_half - 2
+        fixed = size(2 * R) - 2 * unit
+        slots = (size(0) - fixed) // unit
+    finally:
+        lib.cvmm_tuning_set(N.TUNE_WGRAD_CHUNK, 0)
+    assert slots == 2 * R // chunk + 1
+
+
 def test_invalid_arguments_fail_before_launch(lib):
     rc = lib.cvmm_sort_routes(None, 0, 10, 0, 1, None, None, None, None, None, None, None, 0, None)
     assert rc == 1 and b"n_experts" in lib.cvmm_last_error()
