@@ -153,18 +153,19 @@ class _CopyPlan(NamedTuple):
     layout: int  # N.CAST_*_INTERLEAVED bits
     fwd_t: bool
     bwd_t: bool
-    stored: bool
-    cast_n: bool  # kn is a copy
-    casts: bool   # there is a copy to cast
+    stored: bool = False
 
+    @property
+    def cast_n(self) -> bool:
+        return self.want_n and not self.stored
 
-def _new_plan(want_t: bool, want_n: bool, layout: int, fwd_t: bool, bwd_t: bool, stored: bool = False) -> _CopyPlan:
-    cast_n = want_n and not stored
-    return _CopyPlan(want_t, want_n, layout, fwd_t, bwd_t, stored, cast_n, want_t or cast_n)
+    @property
+    def casts(self) -> bool:
+        return self.want_t or self.cast_n
 
 
 # an eager call takes its plan from the few dozen there are
-_kept_plan = functools.lru_cache(None)(_new_plan)
+_kept_plan = functools.lru_cache(None)(_CopyPlan)
 
 
 def _sort_routes_cast(raw_flat: torch.Tensor, n_experts: int, top_k: int, cast, counted_ws=None):
@@ -221,7 +222,7 @@ def _plan_copies(keys: torch.Tensor, op: torch.dtype, n_routes: int, top_k: int,
                  and _topk_dense(T, E, d_out, d_in, top_k, op_id))
     if _compiling():
         fwd_t, bwd_t = not fwd_dense, bwd_dense
-        return _new_plan(fwd_t or (need_grad_input and bwd_t), (not fwd_t) or (need_grad_input and not bwd_t),
+        return _CopyPlan(fwd_t or (need_grad_input and bwd_t), (not fwd_t) or (need_grad_input and not bwd_t),
                          0, fwd_t, bwd_t)
     return _eager_plan(keys, op, n_routes, fwd_dense, bwd_dense, need_grad_input, weighted and cvmm_atomic_reduce)
 
